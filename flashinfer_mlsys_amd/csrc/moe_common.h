@@ -43,10 +43,11 @@ static_assert(sizeof(DispatchHeader) == 512, "header is 512 bytes");
 // One MFMA over a full 128-wide K block: D(16x16 fp32) = A(16x128 e4m3) * B(128x16 e4m3).
 // Lane l holds row (l % 16) of A / column (l % 16) of B and the 32 K values
 // [32*(l/16), 32*(l/16)+32); the result holds rows 4*(l/16)+r, column l % 16.
-// E8M0 scale 127 is 2^0: block scales are applied in fp32 by the caller.
+// With both scale operands constant zero the compiler selects the unscaled form (half the
+// encoding, no scale registers): block scales are applied in fp32 by the caller.
 __device__ __forceinline__ v4f mfma_fp8_k128(const v8i& a, const v8i& b) {
   v4f z = {0.f, 0.f, 0.f, 0.f};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 127, 0, 127);
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 0, 0, 0);
 }
 
 // D += A(16x32 bf16) * B(32x16 bf16); lane l holds row/column l % 16 and
@@ -80,11 +81,17 @@ __device__ __forceinline__ v8h fp8x8_to_f16x8(uint32_t w0, uint32_t w1) {
 // its fp32 accumulators by 2^8 together with the weight block scale.
 constexpr float C_STORE_SCALE = 1.0f / 256.0f;
 constexpr float C_LOAD_SCALE = 256.0f;
-__device__ __forceinline__ uint16_t c_encode(float c) {
-  const float x = c * C_STORE_SCALE;  // exact: a power of two
-  const float y = x != x ? x : fminf(fmaxf(x, -65504.0f), 65504.0f);
-  return __builtin_bit_cast(uint16_t, (_Float16)y);  // round to nearest even
+// Two values to fp16, the first in the low half: round to nearest even, saturating, NaN
+// kept (the IEEE minimum / maximum propagate it).
+__device__ __forceinline__ uint32_t f16x2_sat(float a, float b) {
+  const v2h h = __builtin_convertvector((v2f{a, b}), v2h);
+  const v2h hi = {(_Float16)65504.0f, (_Float16)65504.0f};
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_maximum(__builtin_elementwise_minimum(h, hi), -hi));
 }
+__device__ __forceinline__ uint32_t c_encode2(float a, float b) {
+  return f16x2_sat(a * C_STORE_SCALE, b * C_STORE_SCALE);  // exact: a power of two
+}
+__device__ __forceinline__ uint16_t c_encode(float c) { return (uint16_t)c_encode2(c, c); }
 
 // Barrier for LDS traffic only. __syncthreads() also orders global memory, and
 // since global stores count in vmcnt like loads, it waits for every load in

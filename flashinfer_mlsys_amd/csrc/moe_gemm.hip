@@ -51,8 +51,11 @@ __device__ __forceinline__ v8i load_v8i(const uint8_t* p) {
   return r;
 }
 
+// silu(x2) * x1 in fp32 from the hardware's exp2 and reciprocal (1 ulp each): a few fp32
+// ulps, against the 2^-12 relative rounding of the fp16 result.
 __device__ __forceinline__ float silu_mul(float x1, float x2) {
-  return (x2 / (1.0f + expf(-x2))) * x1;
+  constexpr float LOG2E = 1.44269504088896340736f;
+  return x2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x2 * -LOG2E)) * x1;
 }
 
 // Swizzled 16 x 128 B e4m3 fragment (2 KB), written by two direct loads of 8
@@ -801,36 +804,42 @@ constexpr int FRAG_BYTES = 2048;
 // wn) owns the 16-row fragments 4 mt + wm (mt < 4; the groups interleave, so a
 // partly filled tile spreads its valid fragments evenly over the waves) against
 // 4 X1 and 4 X2 column fragments: 32 MFMAs of 16x16x128 per K block into 128
-// fp32 accumulators. Fragments past the valid rows are skipped, and so are the
-// direct loads of activation rows past them.
+// fp32 accumulators. Fragments past the valid rows are skipped.
 //
-// Every wave computes, and every wave moves an eighth of each K block global ->
-// LDS with direct loads into a ring of stages. An item with more than 128 valid
-// rows uses 2 stages of 66 KB (the loads of block kb+1 fly while kb computes);
-// one with at most 128 uses 3 stages of 50 KB (its activation part is half as
-// large), so the loads of kb+2 fly while kb computes: such items do little MFMA
-// work per block and would otherwise wait for an HBM round trip every block.
-// The direct loads are issued from inline asm: the compiler does not track them,
-// so it puts no wait for them before the fragment reads of the other stages (for
-// the builtin it waits for every direct load in flight before any LDS read, which
-// is why a design built on the builtin needs loader waves that never read LDS,
-// and loses a third of the register file to them). The kernel waits for its own
-// loads explicitly (s_waitcnt vmcnt) before the barrier that ends every K block.
-// M0, which the direct load takes its LDS address from, is set in the same asm
+// The loads: every wave moves an eighth of each K block global -> LDS with direct
+// buffer loads (rows past the valid ones: an offset out of the resource's range,
+// zeros without a memory access) into a ring of NST stages: 2 stages of 64 KB for
+// items with more than 128 valid rows, 3 of 48 KB for the others (half the
+// activation part). They are issued from inline asm, which the compiler does not
+// track: for the builtin it waits for every direct load in flight before any LDS
+// read. M0, which holds a direct load's LDS address, is set in the same asm
 // statement; nothing else in this kernel uses M0.
 //
-// The waves issue their direct loads at two points of the block: waves 0-3 at its
-// top, waves 4-7 halfway through their MFMAs, so the two waves of a SIMD (w,
-// w + 4) take turns. Issued by all waves at the top of the block they held every
-// wave there for ~1,000 clk (the CU moves about 64 B/clk from L2 into LDS, 64 KB
-// per block); split, the loads of one half run beside the other half's MFMAs,
-// and a wave stalled on a full load queue leaves its SIMD to the other wave.
+// The schedule of a block (one accumulator set, four column groups c = 0..3):
+//  * the weight fragments of group c + 1 are read from LDS while group c computes,
+//    and the activation fragments are replaced by the next block's one by one
+//    during group 3, each right after its last product, so no MFMA waits for the
+//    LDS latency;
+//  * two barriers: Y after group 0 (the block's activations and groups 0 and 1
+//    are read: their part of the stage is free) and X after group 2 (groups 2 and 3
+//    are read). Block kb + NST's loads go out as the parts become free, one after
+//    each pair of products, since a wave stalls on issuing a load while the CU's
+//    load path is busy; each load has at least NST - 1 blocks to arrive, and the
+//    waits before the barriers count (vmcnt) and never drain;
+//  * the four fp32 FMAs of a product (s_act[row, kb] * s_w[block, kb] times it)
+//    follow the next product's MFMA, pinned there with sched_barrier: left to
+//    itself the compiler puts them right behind their own MFMA and waits;
+//  * the waves' issue priority falls as they advance between two barriers, so the
+//    two waves of a SIMD alternate instead of running one after the other (the
+//    oldest wave wins ties), and one computes while the other waits for LDS.
 //
-// Per K block and row the fp32 factors s_act[row, kb] * s_w[X1 or X2 block, kb]
-// are formed once (wave w: row 64 (w % 4) + lane, X1 for w < 4, X2 above) and
-// stored in the stage beside the operands as (X1, X2) pairs, one block ahead; the
-// activation scales and the two weight block scales arrive two blocks ahead by
-// direct loads into a small LDS buffer.
+// Measured (GEMM1 alone, us, against the version that loaded a whole block between
+// two barriers and read each block's fragments after its barrier): skewed T=4096
+// (24.7k pairs, 227 rows a tile) 807 -> 660, T=14,107 571 -> 498, T=8192 393 -> 331,
+// T=3001 218 -> 191, T=901 165 -> 165 (5.7 TB/s of weights). On full tiles a block
+// takes 3,000 clk (2,176 of MFMAs; 2,950 with every MFMA taken out, the load path's
+// ~22 B/clk per CU), and the clock falls to 1.9-2.0 GHz: MFMAs alone on such data
+// run at 3.7 PFLOP/s, the card's power limit.
 // ---------------------------------------------------------------------------
 constexpr int P1_BM = 256;
 constexpr int P1_BNP = 128;
@@ -838,18 +847,19 @@ constexpr int P1_NT = I / P1_BNP;          // 16 column-pair tiles
 constexpr int P1_WAVES = 8;
 constexpr int P1_THREADS = 64 * P1_WAVES;
 constexpr int P1_B_BYTES = 2 * P1_BNP * BLK;  // 32 KB: 16 weight fragments (0-7 X1, 8-15 X2)
-constexpr int P1_F_BYTES = 2 * P1_BM * 4;     // (X1, X2) factor pairs of the 256 rows
+// LDS of an NST-stage ring: the stages (activation rows, then the 16 weight fragments),
+// NST buffers of activation scales, the (X1, X2) weight scales of the item's blocks.
 template <int NST>
-struct P1Ring {  // the stage layout of an NST-stage ring
-  static constexpr int A_BYTES = (NST == 2 ? P1_BM : P1_BM / 2) * BLK;
-  static constexpr int B_OFF = A_BYTES;
-  static constexpr int F_OFF = A_BYTES + P1_B_BYTES;
-  static constexpr int STAGE = F_OFF + P1_F_BYTES;
-  static constexpr int BYTES = NST * STAGE;
+struct P1Ring {
+  static constexpr int ROWS = NST == 2 ? P1_BM : P1_BM / 2;
+  static constexpr int B_OFF = ROWS * BLK;
+  static constexpr int STAGE = B_OFF + P1_B_BYTES;
+  static constexpr int SA_OFF = NST * STAGE;
+  static constexpr int SW_OFF = SA_OFF + NST * ROWS * 4;
+  static constexpr int BYTES = SW_OFF + 512;
+  static constexpr int NA = ROWS / 128;  // activation loads of a wave in each of its two steps
 };
-constexpr int P1_SA_OFF = P1Ring<2>::BYTES > P1Ring<3>::BYTES ? P1Ring<2>::BYTES : P1Ring<3>::BYTES;
-constexpr int P1_SA_BUF = P1_BM * 4 + 16;  // activation scales of the 256 rows, then the X1 and X2 weight scales
-constexpr int P1_LDS = P1_SA_OFF + 2 * P1_SA_BUF;
+constexpr int P1_LDS = P1Ring<2>::BYTES > P1Ring<3>::BYTES ? P1Ring<2>::BYTES : P1Ring<3>::BYTES;
 // 32-item blocks: 4 row tiles x 8 column tiles, or 2 x 16 when no expert has more
 // than one row tile (every block then holds all column tiles of 2 experts, whose
 // activation rows its 32 workgroups share; with several row tiles per expert the
@@ -874,14 +884,9 @@ __device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p);
 }
 
-// Direct global -> LDS loads of 16 (4) B per lane from base + voff; lane l's bytes
-// land at lds + 16 l (4 l). Untracked by the compiler (see above). s_nop 4 covers
-// the wait states after an M0 write and after a VALU write of the base SGPRs.
-__device__ __forceinline__ void dma16(const void* base, uint32_t voff, const uint8_t* lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base),
-               "s"(lds_addr(lds))
-               : "memory");
-}
+// Direct global -> LDS load of 4 B per lane from base + voff; lane l's bytes land at
+// lds + 4 l. Untracked by the compiler (see above). s_nop 4 covers the wait states
+// after an M0 write and after a VALU write of the base SGPRs.
 __device__ __forceinline__ void dma4(const void* base, uint32_t voff, const uint8_t* lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base),
                "s"(lds_addr(lds))
@@ -956,227 +961,257 @@ __device__ __forceinline__ const int32_t* p1_token_ptr(const int32_t* perm_tok, 
 }
 
 struct P1Ctx {
-  const uint8_t* hidden;
-  const float* hscale;
-  int T;
-  const uint8_t* w13;
+  int T;  // row stride of hscale
   const float* s13;
   uint16_t* c_act;
-  int w, lane, wm, wn, fr, kg, flo, fhi, frow, fkind;
+  int w, lane, wm, wn, flo, fhi;
 };
 
-// One wave's loads of one item, as byte offsets: A half fragments 4 w + j (tile
-// rows 32 w + 8 j + l / 8, from hidden) and B half fragments 4 w + j (fragment
-// f = (4 w + j) / 2: X1 rows 128 nt + 16 f + ..., X2 rows for f >= 8, from w13),
-// 16 B chunk (l % 8) ^ (l / 8) ^ half, without the K block's 128 B; the
-// activation-scale row (waves 0-3, from hscale) and the X1 / X2 weight-scale rows
-// (wave 4 lanes 0 / 1, from s13).
+// A raw-buffer resource as four words, for inline asm.
+__device__ __forceinline__ v4i buf_words(const void* base, uint32_t bytes) {
+  const uint64_t b = (uint64_t)(uintptr_t)base;
+  return v4i{(int)(uint32_t)b, (int)(uint32_t)(b >> 32), (int)bytes, 0x00020000};
+}
+
+// Direct buffer -> LDS loads of 16 (4) B per lane from the resource's base + voff +
+// soff; lane l's bytes land at lds + 16 l (4 l), zeros when the offset is out of the
+// resource's range. Untracked by the compiler; s_nop 4 as above.
+__device__ __forceinline__ void bdma16(v4i rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs),
+               "s"(soff), "s"(lds)
+               : "memory");
+}
+__device__ __forceinline__ void bdma4(v4i rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(rs),
+               "s"(soff), "s"(lds)
+               : "memory");
+}
+// This wave's issue priority (a constant after unrolling).
+__device__ __forceinline__ void wave_prio(int p) {
+  switch (p) {
+    case 0: __builtin_amdgcn_s_setprio(0); break;
+    case 1: __builtin_amdgcn_s_setprio(1); break;
+    case 2: __builtin_amdgcn_s_setprio(2); break;
+    default: __builtin_amdgcn_s_setprio(3); break;
+  }
+}
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// v as a value the compiler cannot trace: what is derived from it is computed where it
+// is used, not once per kernel into registers that the K loops need.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// One wave's loads of one item: the buffer resources (activations, weights,
+// activation scales) and the lane's offsets. Activation half fragments (8 rows)
+// 8 NA (j / NA) + NA w + j % NA; of W13 the two halves of fragment (w % 2) +
+// 4 (w / 2) (column groups 0 and 1; + 2: groups 2 and 3); lane l takes row l / 8,
+// 16 B chunk (l % 8) ^ (l / 8) ^ half.
 struct P1Src {
-  uint32_t a[4], b[4];
-  int na;          // A half fragments holding valid rows (uniform)
-  uint32_t sa;     // activation scale of row 64 w + lane (waves 0-3)
-  uint32_t sw;     // weight-scale row (wave 4, lanes 0 and 1)
+  v4i ra, rb, rs;
+  uint32_t a[4], b[2], sa;
 };
 
+template <int NST>
 __device__ __forceinline__ void p1_src(const P1Ctx& x, const int32_t* perm_tok, const P1Item& it, P1Src& s) {
-  const int rr = x.lane >> 3;
-  int tok[4], tsa;
-  ld_sync4(p1_token_ptr(perm_tok, it, 32 * x.w + rr), p1_token_ptr(perm_tok, it, 32 * x.w + 8 + rr),
-           p1_token_ptr(perm_tok, it, 32 * x.w + 16 + rr), p1_token_ptr(perm_tok, it, 32 * x.w + 24 + rr), tok[0],
-           tok[1], tok[2], tok[3]);
-  ld_sync1(p1_token_ptr(perm_tok, it, x.frow), tsa);
+  constexpr int NA = P1Ring<NST>::NA;
+  const int lane = opaque(x.lane), rr = lane >> 3, w = x.w;
+  int row[4], tok[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int h = 4 * x.w + j, half = h & 1, c = (x.lane & 7) ^ rr ^ half;
-    s.a[j] = (uint32_t)tok[j] * H + c * 16;
-    const int f = h >> 1;
-    const int row = (f < 8 ? it.nt * P1_BNP + 16 * f : I + it.nt * P1_BNP + 16 * (f - 8)) + 8 * half + rr;
-    s.b[j] = ((uint32_t)it.e * N1 + row) * H + c * 16;
+  for (int j = 0; j < 4; ++j)  // step j / NA: half fragments 8 NA (j / NA) + NA w + j % NA
+    row[j] = 8 * (8 * NA * (j / NA) + NA * w + j % NA) + rr;
+  ld_sync4(p1_token_ptr(perm_tok, it, row[0]), p1_token_ptr(perm_tok, it, row[1]), p1_token_ptr(perm_tok, it, row[2]),
+           p1_token_ptr(perm_tok, it, row[3]), tok[0], tok[1], tok[2], tok[3]);
+#pragma unroll
+  for (int j = 0; j < 2 * NA; ++j) {
+    const int half = NA == 2 ? (j & 1) : (w & 1);
+    s.a[j] = row[j] < it.valid ? (uint32_t)tok[j] * H + (((lane & 7) ^ rr ^ half) << 4) : 0xFFFFFF00u;
   }
-  s.na = min(4, max(0, (it.valid - 32 * x.w + 7) / 8));
+  const int i = w >> 1, wrow = (i >> 1) * I + it.nt * P1_BNP + 64 * (i & 1) + 16 * (w & 1);
+#pragma unroll
+  for (int half = 0; half < 2; ++half)
+    s.b[half] = ((uint32_t)it.e * N1 + wrow + 8 * half + rr) * H + (((lane & 7) ^ rr ^ half) << 4);
+  int tsa;
+  ld_sync1(p1_token_ptr(perm_tok, it, (64 * w + lane) & (P1_BM - 1)), tsa);
   s.sa = (uint32_t)tsa * 4;
-  s.sw = ((uint32_t)it.e * NB_N1 + ((x.lane & 1) ? NB_I + it.nt : it.nt)) * NB_H * 4;
 }
 
-// Scales of block kb into SA buffer kb % 2.
-__device__ __forceinline__ void p1_scales(const P1Ctx& x, const P1Src& s, uint8_t* lds, int kb) {
-  uint8_t* sb = lds + P1_SA_OFF + (kb & 1) * P1_SA_BUF;
-  if (x.w < 4) dma4(x.hscale + (size_t)kb * x.T, s.sa, sb + 256 * x.w);
-  if (x.w == 4 && x.lane < 2) dma4(x.s13 + kb, s.sw, sb + P1_BM * 4);
-}
-
-// This wave's factor of block kb (its scales are in SA buffer kb % 2) into the
-// factor region f of the block's stage.
-__device__ __forceinline__ void p1_factor(const P1Ctx& x, const uint8_t* lds, uint8_t* f, int kb) {
-  const uint8_t* sb = lds + P1_SA_OFF + (kb & 1) * P1_SA_BUF;
-  const float sa = reinterpret_cast<const float*>(sb)[x.frow];
-  const float sw = reinterpret_cast<const float*>(sb + P1_BM * 4)[x.fkind];
-  reinterpret_cast<float*>(f)[2 * x.frow + x.fkind] = sa * sw;
-}
-
-// This wave's operand loads of block kb into the stage at st.
-template <int B_OFF>
-__device__ __forceinline__ void p1_operands(const P1Ctx& x, const P1Src& s, uint8_t* st, int kb) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (j < s.na) dma16(x.hidden + kb * BLK, s.a[j], st + (4 * x.w + j) * 1024);
-    dma16(x.w13 + kb * BLK, s.b[j], st + B_OFF + (4 * x.w + j) * 1024);
-  }
-}
-
-// One K block of a wave: NMT valid token fragments (4 mt + wm) x 4 X1 + 4 X2 weight
-// fragments, accumulated with the stage's factors. The weight fragment is the
-// MFMA's first operand, so lane l's four results are weight columns 4 (l / 16) + r
-// of one token (l % 16), and the token's two factors (X1, X2) are one 8-byte LDS
-// read per fragment. The next block's operand loads (load(), when any) go out
-// before column group DMA_AT; for DMA_AT > 0 empty asm statements that read the
-// earlier groups' accumulators come first: asm volatile statements keep their
-// order, so those groups' MFMAs stay above the loads (without them the
-// instruction DAG sinks every MFMA below the loads).
-template <int NMT, int DMA_AT, int B_OFF, int F_OFF, typename Load>
-__device__ __forceinline__ void p1_block(const P1Ctx& x, const uint8_t* st, v4f (&au)[4][4], v4f (&ag)[4][4],
-                                         const Load& load) {
-  v8i a[NMT];
-  v2f f[NMT];
-#pragma unroll
-  for (int mt = 0; mt < NMT; ++mt) {
-    a[mt] = lds_frag_sw(st + (4 * mt + x.wm) * FRAG_BYTES, x.flo, x.fhi);
-    f[mt] = *reinterpret_cast<const v2f*>(st + F_OFF + ((4 * mt + x.wm) * 16 + x.fr) * 8);
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    if (c == DMA_AT) {
-#pragma unroll
-      for (int cc = 0; cc < DMA_AT; ++cc)
-#pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) asm volatile("" ::"v"(au[mt][cc]), "v"(ag[mt][cc]));
-      load();
-    }
-    const v8i bu = lds_frag_sw(st + B_OFF + (4 * x.wn + c) * FRAG_BYTES, x.flo, x.fhi);
-    const v8i bg = lds_frag_sw(st + B_OFF + (8 + 4 * x.wn + c) * FRAG_BYTES, x.flo, x.fhi);
-#pragma unroll
-    for (int mt = 0; mt < NMT; ++mt) {
-      const v4f pu = mfma_fp8_k128(bu, a[mt]);
-      const v4f pg = mfma_fp8_k128(bg, a[mt]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        au[mt][c][r] += pu[r] * f[mt][0];
-        ag[mt][c][r] += pg[r] * f[mt][1];
-      }
-    }
-  }
-}
-
-// s_waitcnt vmcnt(n) for a uniform n in 0..8.
-__device__ __forceinline__ void wait_vm(int n) {
-  switch (n) {
-    case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
-    case 1: asm volatile("s_waitcnt vmcnt(1)" ::: "memory"); break;
-    case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
-    case 3: asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); break;
-    case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
-    case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
-    case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
-    case 7: asm volatile("s_waitcnt vmcnt(7)" ::: "memory"); break;
-    default: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
-  }
-}
-
-// One item on an NST-stage ring (a wave with NMT valid token fragments): the
-// prologue fills stages 0..NST-2 and the scales of blocks 0 and 1, then each
-// block kb computes from stage kb % NST while its waves load block kb + NST - 1.
-// Before the barrier that ends block kb each wave waits for all its loads but
-// those of block kb + NST - 1 (loads complete in order; the scale loads of the
-// block are issued before them), so block kb + 1's operands and kb + 2's scales
-// are in place.
-template <int NMT, int DMA_AT, int NST>
+template <int NMT, int NST>
 __device__ __forceinline__ void p1_run_item(const P1Ctx& x, const P1Item& ic, const P1Src& s, uint8_t* lds) {
   using R = P1Ring<NST>;
+  constexpr int NA = R::NA, NL = 2 * NA + 4;  // direct loads of a wave per block (the scale loads uncounted)
+  const int w = x.w;
+  const uint32_t l0 = lds_addr(lds);
+  const uint32_t fb = R::B_OFF + ((w & 1) + 4 * (w >> 1)) * FRAG_BYTES;
+  auto load_a = [&](int j, int h, int kb, uint32_t st) {
+    bdma16(s.ra, s.a[NA * j + h], kb * BLK, l0 + st + (8 * NA * j + NA * w + h) * 1024);
+  };
+  auto load_b = [&](int c, int h, int kb, uint32_t st) {  // c 0: column groups 0 and 1, 2: groups 2 and 3
+    bdma16(s.rb, s.b[h], kb * BLK + 16 * c * H, l0 + st + fb + c * FRAG_BYTES + h * 1024);
+  };
+  auto load_sa = [&](int kb, int slot) {
+    if (w < R::ROWS / 64) bdma4(s.rs, s.sa, (uint32_t)kb * x.T * 4, l0 + R::SA_OFF + slot * (R::ROWS * 4) + w * 256);
+  };
+  if (w >= 6) {  // the weight scales of the item: word j = block j / 2, X1 / X2
+    const int j = min(64 * (w - 6) + x.lane, 2 * NB_H - 1);
+    dma4(x.s13, (((uint32_t)ic.e * NB_N1 + (j & 1) * NB_I + ic.nt) * NB_H + (j >> 1)) * 4,
+         lds + R::SW_OFF + 256 * (w - 6));
+  }
 #pragma unroll
-  for (int b = 0; b < NST - 1; ++b) p1_operands<R::B_OFF>(x, s, lds + b * R::STAGE, b);
-  p1_scales(x, s, lds, 0);
-  p1_scales(x, s, lds, 1);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  lds_barrier();
-  p1_factor(x, lds, lds + R::F_OFF, 0);
-  lds_barrier();
-
-  v4f au[4][4], ag[4][4];
+  for (int b = 0; b < NST; ++b) {
+    load_sa(b, b);
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int h = 0; h < NA; ++h) load_a(j, h, b, b * R::STAGE);
+      load_b(0, j, b, b * R::STAGE);
+    }
+    load_b(2, 0, b, b * R::STAGE);
+    load_b(2, 1, b, b * R::STAGE);
+  }
+  constexpr int NM = NMT ? NMT : 1;
+  v4f au[NM][4], ag[NM][4], pu[2], pg[2];
+  v2f f[NM], sw;
+  float sa[NM];
+  v8i a[NM], bu[2], bg[2];
+#pragma unroll
+  for (int mt = 0; mt < NMT; ++mt)
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       au[mt][c] = v4f{0.f, 0.f, 0.f, 0.f};
       ag[mt][c] = au[mt][c];
     }
-  const int n_ld = s.na + 4;  // direct loads of this wave per block
-  int cur = 0;
+  pu[1] = pg[1] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto read_b = [&](int c, uint32_t st) {
+    const uint8_t* sb = lds + st + R::B_OFF + (4 * x.wn + c) * FRAG_BYTES;
+    bu[c & 1] = lds_frag_sw(sb, x.flo, x.fhi);
+    bg[c & 1] = lds_frag_sw(sb + 8 * FRAG_BYTES, x.flo, x.fhi);
+  };
+  auto read_a = [&](int mt, uint32_t st) { a[mt] = lds_frag_sw(lds + st + (4 * mt + x.wm) * FRAG_BYTES, x.flo, x.fhi); };
+  auto read_s = [&](int kb, int slot) {
+#pragma unroll
+    for (int mt = 0; mt < NMT; ++mt)
+      sa[mt] = *reinterpret_cast<const float*>(lds + R::SA_OFF + slot * (R::ROWS * 4) + x.wm * 64 + (x.lane & 15) * 4 + mt * 256);
+    sw = *reinterpret_cast<const v2f*>(lds + R::SW_OFF + kb * 8);
+  };
+  // the products in p, times the row's factor, into one accumulator
+  auto fma = [&](v4f& acc, const v4f& p, float fac) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] += p[r] * fac;
+    asm volatile("" : "+v"(acc)::"memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  if constexpr (NMT > 0) {
+    read_b(0, 0);
+#pragma unroll
+    for (int mt = 0; mt < NMT; ++mt) {
+      f[mt] = v2f{0.f, 0.f};
+      read_a(mt, 0);
+    }
+    read_s(0, 0);
+  }
+  uint32_t st = 0;  // stage of block kb
+  int slot = 0;
 #pragma unroll 1
   for (int kb = 0; kb < NB_H; ++kb) {
-    const int nxt = cur == NST - 1 ? 0 : cur + 1;          // stage of block kb + 1
-    const int ld = NST == 2 ? nxt : (nxt == NST - 1 ? 0 : nxt + 1);  // stage of block kb + NST - 1
-    if (kb + 1 < NB_H) p1_factor(x, lds, lds + nxt * R::STAGE + R::F_OFF, kb + 1);
-    if (kb + 2 < NB_H) p1_scales(x, s, lds, kb + 2);
-    const int kl = kb + NST - 1;
-    const bool loading = kl < NB_H;
-    auto load = [&]() {
-      if (loading) p1_operands<R::B_OFF>(x, s, lds + ld * R::STAGE, kl);
-    };
-    if constexpr (NMT > 0) {
-      p1_block<NMT, DMA_AT, R::B_OFF, R::F_OFF>(x, lds + cur * R::STAGE, au, ag, load);
-    } else {
-      load();
-    }
-    if (kb == NB_H - 1) {
-      // SwiGLU and the fp16 C rows (lane l: token row 16 (4 mt + wm) + l % 16, four
-      // consecutive columns from 4 (l / 16) of each of its 4 column fragments)
+    const bool more = kb + NST < NB_H;
+    const int slot1 = slot == NST - 1 ? 0 : slot + 1;
+    const uint32_t st1 = slot1 * R::STAGE;
 #pragma unroll
-      for (int mt = 0; mt < NMT; ++mt) {
-        const int row = (4 * mt + x.wm) * 16 + x.fr;
-        if (row < ic.valid) {
-          uint16_t* dst = x.c_act + (size_t)(ic.seg + ic.m0 + row) * I + ic.nt * P1_BNP + 4 * x.kg;
+    for (int c = 0; c < 4; ++c) {
+      // the group's direct loads, one per step: spread over the MFMAs, since a wave
+      // that issues while the CU's load path is busy stalls its MFMAs as well
+      constexpr int NLD[4] = {0, NA + 1, NA + 1, 2};
+      auto load = [&](int i) {
+        if (!more || i >= NLD[c]) return;
+        if (c == 3) load_b(2, i, kb + NST, st);
+        else if (i == NA) load_b(0, c - 1, kb + NST, st);
+        else load_a(c - 1, i, kb + NST, st);
+        if (c == 1 && i == 0) load_sa(kb + NST, slot);
+      };
+      if constexpr (NMT == 0) {
 #pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            uint2 v;
-            v.x = (uint32_t)c_encode(silu_mul(au[mt][c][0], ag[mt][c][0])) |
-                  ((uint32_t)c_encode(silu_mul(au[mt][c][1], ag[mt][c][1])) << 16);
-            v.y = (uint32_t)c_encode(silu_mul(au[mt][c][2], ag[mt][c][2])) |
-                  ((uint32_t)c_encode(silu_mul(au[mt][c][3], ag[mt][c][3])) << 16);
-            *reinterpret_cast<uint2*>(dst + (4 * x.wn + c) * 16) = v;
+        for (int i = 0; i < NA + 1; ++i) load(i);
+      }
+      if constexpr (NMT > 0) {
+        if (c < 3) read_b(c + 1, st);
+        else read_b(0, st1);
+#pragma unroll
+        for (int mt = 0; mt < NMT; ++mt) {
+          if ((mt & 1) == 0) wave_prio(c == 0 || c == 2 ? (mt < 2 ? 1 : 0) : (mt < 2 ? 3 : 2));
+          const int q = (c * NMT + mt) & 1, pm = mt > 0 ? mt - 1 : NM - 1, pc = mt > 0 ? c : (c + 3) & 3;
+          asm volatile("" : "+v"(a[mt]), "+v"(bu[c & 1]), "+v"(bg[c & 1])::"memory");
+          pu[q] = mfma_fp8_k128(bu[c & 1], a[mt]);
+          asm volatile("" : "+v"(pu[q])::"memory");
+          fma(au[pm][pc], pu[q ^ 1], f[pm][0]);
+          pg[q] = mfma_fp8_k128(bg[c & 1], a[mt]);
+          asm volatile("" : "+v"(pg[q])::"memory");
+          if (c == 3) read_a(mt, st1);
+          fma(ag[pm][pc], pg[q ^ 1], f[pm][1]);
+          load(mt);
+          if (mt == NMT - 1) {
+#pragma unroll
+            for (int i = NMT; i < NLD[c]; ++i) load(i);
+          }
+          if (c == 0 && mt == 0) {
+#pragma unroll
+            for (int m = 0; m < NMT; ++m) f[m] = v2f{sa[m] * sw[0], sa[m] * sw[1]};
           }
         }
+        if (c == 3) read_s(min(kb + 1, NB_H - 1), slot1);
+      }
+      if (c == 0) {  // this block's groups 0 and 1 and activations are read; its groups 2 and 3 are in place
+        const int r = NB_H - 1 - kb;
+        if (r >= NST - 1) wait_vmcnt<(NST - 1) * NL>();
+        else if (r == 1) wait_vmcnt<NL>();
+        else wait_vmcnt<0>();
+        lds_barrier();
+      }
+      if (c == 2) {  // this block is read; the next block's activations and groups 0 and 1 are in place
+        const int r = NB_H - 1 - kb;
+        if (r >= NST) wait_vmcnt<(NST - 1) * NL>();
+        else if (r == 2) wait_vmcnt<NL + 2>();
+        else wait_vmcnt<2>();
+        lds_barrier();
       }
     }
-    if (NST == 2 || !loading)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else
-      wait_vm(n_ld);
-    lds_barrier();
-    cur = nxt;
+    slot = slot1;
+    st = st1;
   }
-}
-
-template <int DMA_AT>
-__device__ __forceinline__ void p1_dispatch(const P1Ctx& x, const P1Item& ic, const P1Src& s, uint8_t* lds) {
-  const int nf = (ic.valid + 15) / 16;
-  const int nmt = nf > x.wm ? (nf - x.wm + 3) / 4 : 0;
-  if (ic.valid > P1_BM / 2) {  // nf >= 9: nmt >= 2
-    switch (nmt) {
-      case 2: p1_run_item<2, DMA_AT, 2>(x, ic, s, lds); break;
-      case 3: p1_run_item<3, DMA_AT, 2>(x, ic, s, lds); break;
-      default: p1_run_item<4, DMA_AT, 2>(x, ic, s, lds); break;
-    }
-  } else {  // nf <= 8: nmt <= 2
-    switch (nmt) {
-      case 0: p1_run_item<0, DMA_AT, 3>(x, ic, s, lds); break;
-      case 1: p1_run_item<1, DMA_AT, 3>(x, ic, s, lds); break;
-      default: p1_run_item<2, DMA_AT, 3>(x, ic, s, lds); break;
+  lds_barrier();
+  if constexpr (NMT > 0) {
+    fma(au[NM - 1][3], pu[(4 * NMT - 1) & 1], f[NM - 1][0]);
+    fma(ag[NM - 1][3], pg[(4 * NMT - 1) & 1], f[NM - 1][1]);
+  }
+  const int el = opaque(x.lane), fr = el & 15, kg = el >> 4;
+#pragma unroll
+  for (int mt = 0; mt < NMT; ++mt) {
+    const int row = (4 * mt + x.wm) * 16 + fr;
+    if (row < ic.valid) {
+      uint16_t* dst = x.c_act + (size_t)(ic.seg + ic.m0 + row) * I + ic.nt * P1_BNP + 4 * kg;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        uint2 v;
+        v.x = c_encode2(silu_mul(au[mt][c][0], ag[mt][c][0]), silu_mul(au[mt][c][1], ag[mt][c][1]));
+        v.y = c_encode2(silu_mul(au[mt][c][2], ag[mt][c][2]), silu_mul(au[mt][c][3], ag[mt][c][3]));
+        *reinterpret_cast<uint2*>(dst + (4 * x.wn + c) * 16) = v;
+      }
     }
   }
 }
 
 __global__ __launch_bounds__(P1_THREADS, 1) void gemm1_prefill_kernel(
-    const uint8_t* __restrict__ hidden, const float* __restrict__ hscale, int T, const uint8_t* __restrict__ w13,
+    const uint8_t* __restrict__ hidden, const float* __restrict__ hscale, int T, int n_tok, const uint8_t* __restrict__ w13,
     const float* __restrict__ s13, const DispatchHeader* __restrict__ hdr, const int32_t* __restrict__ perm_tok,
     uint16_t* __restrict__ c_act) {
   extern __shared__ __attribute__((aligned(16))) uint8_t p1_lds[];
@@ -1184,26 +1219,34 @@ __global__ __launch_bounds__(P1_THREADS, 1) void gemm1_prefill_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   build_tile_map<P1_BM>(hdr, map);
   P1Ctx x;
-  x.hidden = hidden; x.hscale = hscale; x.T = T; x.w13 = w13; x.s13 = s13; x.c_act = c_act;
+  x.T = T; x.s13 = s13; x.c_act = c_act;
   x.w = __builtin_amdgcn_readfirstlane(tid >> 6);
   x.lane = lane;
-  x.wm = x.w & 3; x.wn = x.w >> 2; x.fr = lane & 15; x.kg = lane >> 4;
+  x.wm = x.w & 3; x.wn = x.w >> 2;
   frag_sw_offsets(lane, x.flo, x.fhi);
-  x.frow = 64 * (x.w & 3) + lane;  // the factor row this wave forms
-  x.fkind = x.w >> 2;              // 0: X1, 1: X2
   const int total = __builtin_amdgcn_readfirstlane(map.total_m) * P1_NT, G = gridDim.x;
   const int slot = xcd_remap(blockIdx.x, G);
   const bool one_tile = __builtin_amdgcn_ballot_w64((lane < E_LOCAL ? map.cnt[lane] : 0) > P1_BM) == 0;  // uniform
+  P1Src ps;
+  ps.ra = buf_words(hidden, (uint32_t)n_tok * H);
+  ps.rb = buf_words(w13, (uint32_t)E_LOCAL * N1 * H);
+  ps.rs = buf_words(hscale, ((uint32_t)(NB_H - 1) * T + n_tok) * 4);
 #pragma unroll 1
   for (int r = 0;; ++r) {
     P1Item ic;
     if (!p1_item(map, r, slot, G, total, one_tile, ic)) break;
-    P1Src s;
-    p1_src(x, perm_tok, ic, s);
-    if (x.w < 4)
-      p1_dispatch<0>(x, ic, s, p1_lds);
-    else
-      p1_dispatch<2>(x, ic, s, p1_lds);
+    const int nf = (ic.valid + 15) / 16, nmt = nf > x.wm ? (nf - x.wm + 3) / 4 : 0;
+    if (ic.valid > P1_BM / 2) {  // nf >= 9: nmt >= 2
+      p1_src<2>(x, perm_tok, ic, ps);
+      if (nmt == 2) p1_run_item<2, 2>(x, ic, ps, p1_lds);
+      else if (nmt == 3) p1_run_item<3, 2>(x, ic, ps, p1_lds);
+      else p1_run_item<4, 2>(x, ic, ps, p1_lds);
+    } else {  // nf <= 8: nmt <= 2
+      p1_src<3>(x, perm_tok, ic, ps);
+      if (nmt == 0) p1_run_item<0, 3>(x, ic, ps, p1_lds);
+      else if (nmt == 1) p1_run_item<1, 3>(x, ic, ps, p1_lds);
+      else p1_run_item<2, 3>(x, ic, ps, p1_lds);
+    }
   }
 }
 
@@ -1685,7 +1728,7 @@ hipError_t launch_gemm2_decode(const uint16_t* c_act, const uint8_t* w2, const f
   return hipGetLastError();
 }
 
-hipError_t launch_gemm1_prefill(const uint8_t* hidden, const float* hscale, int T, const uint8_t* w13,
+hipError_t launch_gemm1_prefill(const uint8_t* hidden, const float* hscale, int T, int n_tok, const uint8_t* w13,
                                const float* s13, const DispatchHeader* hdr, const int32_t* perm_tok,
                                uint16_t* c_act, int grid, hipStream_t stream) {
   static PerDeviceOnce<hipError_t> once;
@@ -1694,7 +1737,7 @@ hipError_t launch_gemm1_prefill(const uint8_t* hidden, const float* hscale, int 
                                            hipFuncAttributeMaxDynamicSharedMemorySize, P1_LDS); },
            e);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(gemm1_prefill_kernel, dim3(grid), dim3(P1_THREADS), P1_LDS, stream, hidden, hscale, T, w13,
+  hipLaunchKernelGGL(gemm1_prefill_kernel, dim3(grid), dim3(P1_THREADS), P1_LDS, stream, hidden, hscale, T, n_tok, w13,
                      s13, hdr, perm_tok, c_act);
   return hipGetLastError();
 }
