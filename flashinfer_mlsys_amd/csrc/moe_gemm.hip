@@ -1584,6 +1584,356 @@ __global__ __launch_bounds__(W2_THREADS, 1) void gemm2_loader_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// GEMM2 (+ routing weight), prefill shape from WIDE_MIN_TOKENS tokens: items of 256
+// rows x 256 output columns, 8 waves as 2 (rows) x 4 (columns), each 128 x 64 as 8 x 4
+// tiles of the fp16 16x16x32 MFMA (1.87 PFLOP/s on such data against 1.72 for the
+// 32x32x16 form: the card is power-limited, 2.05 against 1.80 GHz). The loader kernel's
+// 128 x 256 items with 64 x 64 per wave read 1.5 times as many LDS bytes per product
+// and leave the 8 compute waves to wait for LDS at every block.
+//
+//  * The weight is the MFMA's first operand, so a lane's four results are four columns
+//    of one token: one routing weight per lane and row fragment, and after a 4 x 4
+//    transposition over the lane groups (permlane swaps) two 16 B stores per fragment.
+//  * Weight block scales: the accumulators are kept in units of the current K block's
+//    scale, rescaled by the ratio of the two scales on entering a block, so the MFMAs
+//    add straight into them (no second set of accumulators). This needs scales within
+//    a factor of 2^40 of each other and of usual size (checked per item and wave); any
+//    others (zeros, say) take the general path, which scales each product.
+//  * LDS: the activations as units of 128 rows x half a K block (64 fp16, a 128 B
+//    line) in 5 slots, W2 as whole K blocks in 2. A step computes one unit: 4 row
+//    fragments x 4 column fragments x 2 MFMAs, with one barrier at its end. Step m
+//    loads unit m + 4 into the slot that step m - 1 freed, and W2's block kb + 2 goes out
+//    in the second half of block kb, whose W2 is then in registers. The waits count
+//    and never drain, across items too: the next item's first blocks load during the
+//    last ones (with no next item the resources' range is 0: zeros, no traffic).
+//  * Within a step each row fragment is read one fragment ahead, W2's next half is
+//    widened in place of the fragments just used up, and the vector instructions sit
+//    between the MFMAs. Wave priorities fall within a step, so the two waves of a
+//    SIMD alternate row fragments.
+//
+// W2's K order: the MFMA step k of half h takes, in lane group g, K = 64 h + 16 g + 8 k +
+// [0, 8) in both operands: one 16 B chunk (4 h + g) of a W2 row per half, chunk 2 g + k of
+// an activation row's half. W2's chunks are placed at position 2 g + h so that both kinds
+// of fragment read are free of bank conflicts.
+//
+// Measured against the loader kernel (whole calls, us): skewed T=4096 1,500 -> 1,400,
+// T=14,107 1,086 -> 1,005, T=4096 451 -> 430, T=3001 389 -> 385; GEMM2 alone at T=2500
+// 151 -> 162, T=2000 129 -> 137, T=901 101 -> 126: most experts there have fewer than 100
+// rows, whose half-empty items cost more than the loader kernel's 64- and 128-row ones.
+// A block takes 5,650 clk on full items (4,608 of MFMAs).
+// ---------------------------------------------------------------------------
+constexpr int W_BM = 256, W_BN = 256;
+constexpr int W_NT = H / W_BN;                // 28 column tiles
+constexpr int W_WAVES = 8, W_THREADS = 64 * W_WAVES;
+constexpr int W_AREG = 128 * 128;             // activation region: 128 rows x half a K block (64 fp16)
+constexpr int W_ASLOTS = 5;
+constexpr int W_BSLOT = W_BN * BLK;           // 32 KB
+constexpr int W_B_OFF = W_ASLOTS * W_AREG;
+constexpr int W_PW_OFF = W_B_OFF + 2 * W_BSLOT;   // routing weights of the item's rows, two buffers
+constexpr int W_S_OFF = W_PW_OFF + 2 * W_BM * 4;  // the item's two scale rows, two buffers of 64 floats
+constexpr int W_LDS = W_S_OFF + 2 * 256;
+static_assert(W_LDS + (int)sizeof(TileMap) <= 160 * 1024, "LDS");
+
+struct WItem {
+  int e, m0, cnt, seg, nt, valid;
+};
+__device__ __forceinline__ bool w_item(const TileMap& map, int r, int slot, int G, int total, WItem& it) {
+  const int i = snake_item(r, slot, G);
+  if (i >= total) return false;
+  const int id = block_order_item(i, map.total_m, W_NT);
+  const int k = id / W_NT;
+  int e, m0;
+  tile_row<W_BM>(map, k, e, m0);
+  it.e = __builtin_amdgcn_readfirstlane(e);
+  it.m0 = __builtin_amdgcn_readfirstlane(m0);
+  it.nt = __builtin_amdgcn_readfirstlane(id - k * W_NT);
+  it.cnt = __builtin_amdgcn_readfirstlane(map.cnt[it.e]);
+  it.seg = __builtin_amdgcn_readfirstlane(map.seg[it.e]);
+  it.valid = min(W_BM, it.cnt - it.m0);
+  return true;
+}
+
+struct WCtx {
+  const uint16_t* c_act;
+  const uint8_t* w2;
+  const float *s2, *perm_w;
+  uint16_t* partial;
+  uint8_t* lds;
+  uint32_t l0;
+  int w, lane, wm, wn, flo, fhi;
+  uint32_t va, vb;  // this lane's offset in an 8-row piece of the activations, of W2
+};
+// The same in the second piece of a fragment: 8 rows on, position parity flipped.
+__device__ __forceinline__ uint32_t w_va1(const WCtx& x) { return ((uint32_t)opaque((int)x.va) ^ 16u) + 8 * I * 2; }
+__device__ __forceinline__ uint32_t w_vb1(const WCtx& x) { return ((uint32_t)opaque((int)x.vb) ^ 64u) + 8 * I; }
+
+struct WSrc {  // an item's operands as buffer resources (range 0: no item, zeros without memory access)
+  v4i a, b, pw, s;
+};
+__device__ __forceinline__ WSrc w_src(const WCtx& x, const WItem& it, bool have) {
+  WSrc s;
+  s.a = buf_words(x.c_act + (size_t)(it.seg + it.m0) * I, have ? (uint32_t)it.valid * I * 2 : 0u);
+  s.b = buf_words(x.w2 + ((size_t)it.e * H + it.nt * W_BN) * I, have ? (uint32_t)W_BN * I : 0u);
+  s.pw = buf_words(x.perm_w + it.seg + it.m0, have ? (uint32_t)it.valid * 4 : 0u);
+  s.s = buf_words(x.s2 + ((size_t)it.e * NB_H + 2 * it.nt) * NB_I, have ? 2u * NB_I * 4 : 0u);
+  return s;
+}
+
+// This wave's loads of activation unit (kb, q): rows 128 (q % 2) + 16 w .., K half q / 2.
+__device__ __forceinline__ void w_load_a(const WCtx& x, v4i rs, int kb, int q, int slot) {
+  const uint32_t so = (uint32_t)((q & 1) * 128 + 16 * x.w) * (I * 2) + kb * 256 + (q >> 1) * 128;
+  const uint32_t d = x.l0 + slot * W_AREG + x.w * 2048;
+  bdma16(rs, x.va, so, d);
+  bdma16(rs, w_va1(x), so, d + 1024);
+}
+// This wave's loads of W2 fragment 2 w + f of block kb.
+__device__ __forceinline__ void w_load_b(const WCtx& x, v4i rs, int kb, int f, int slot) {
+  const uint32_t so = (uint32_t)(2 * x.w + f) * 16 * I + kb * BLK;
+  const uint32_t d = x.l0 + W_B_OFF + slot * W_BSLOT + (2 * x.w + f) * 2048;
+  bdma16(rs, x.vb, so, d);
+  bdma16(rs, w_vb1(x), so, d + 1024);
+}
+__device__ __forceinline__ void w_load_meta(const WCtx& x, const WSrc& s, int buf) {
+  if (x.w < 4) bdma4(s.pw, (uint32_t)(64 * x.w + x.lane) * 4, 0, x.l0 + W_PW_OFF + buf * (W_BM * 4) + x.w * 256);
+  if (x.w == 4) bdma4(s.s, (uint32_t)x.lane * 4, 0, x.l0 + W_S_OFF + buf * 256);
+}
+
+struct WState {
+  int aslot;  // LDS slot of the unit the next step computes
+  int buf;    // weights and scales buffer of the current item
+};
+
+template <int NI, bool RATIO>
+__device__ __forceinline__ void w_run(const WCtx& x, const WItem& it, const WSrc& cur, const WSrc& nxt, WState& st,
+                                      float ratio, float sc, v4f (&acc)[NI][4], v8h (&b)[4][2], v4i (&raw)[4],
+                                      v8h (&a)[2][2]) {
+#pragma unroll 1
+  for (int kb = 0; kb < NB_I; ++kb) {
+    const v4i ra = kb == NB_I - 1 ? nxt.a : cur.a, rb = kb >= NB_I - 2 ? nxt.b : cur.b;
+    const int ka = kb == NB_I - 1 ? 0 : kb + 1, kbb = (kb + 2) & (NB_I - 1);
+    const float r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ratio), kb));
+    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ratio), (kb + 1) & 15));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int h = q >> 1, ih = q & 1;
+      const uint8_t* as = x.lds + st.aslot * W_AREG;
+      const int ns = st.aslot == W_ASLOTS - 1 ? 0 : st.aslot + 1;
+      const int ls = st.aslot == 0 ? W_ASLOTS - 1 : st.aslot - 1;  // the slot before: free
+      // raw W2 of the next half: (kb, 1) in step 1, (kb + 1, 0) in step 3
+      if (ih == 1) {
+        const uint8_t* bs = x.lds + W_B_OFF + ((kb + h) & 1) * W_BSLOT + (4 * x.wn) * 2048;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const v4i*>(bs + j * 2048 + (h ? x.flo : x.fhi));
+      }
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) {
+        const int i = 4 * ih + ii, p = RATIO ? ii & 1 : 0;
+        wave_prio(3 - ii);
+        // the next row fragment (of the next step's unit at the end)
+        if constexpr (RATIO) {
+          const uint8_t* an = ii < 3 ? as + (2 * (ii + 1) + x.wm) * 2048 : x.lds + ns * W_AREG + x.wm * 2048;
+          const bool need = ii < 3 ? i + 1 < NI : (ih == 0 ? 4 < NI : true);
+          if (need) {
+            a[p ^ 1][0] = *reinterpret_cast<const v8h*>(an + x.flo);
+            a[p ^ 1][1] = *reinterpret_cast<const v8h*>(an + x.fhi);
+          }
+        } else if (i < NI) {  // (the general path: this fragment itself, no registers for the next)
+          a[0][0] = *reinterpret_cast<const v8h*>(as + (2 * ii + x.wm) * 2048 + x.flo);
+          a[0][1] = *reinterpret_cast<const v8h*>(as + (2 * ii + x.wm) * 2048 + x.fhi);
+        }
+        // The vector work goes between the MFMAs (16 clk each) two or four
+        // instructions at a time, ahead of its use: the rescaling of the row fragment
+        // that enters the K block next, and the widening of W2's next half in place of
+        // the fragments just used up.
+        const bool mul_next = h == 0 && (ii < 3 || ih == 0) && i + 1 < NI;
+        const bool mul_first = q == 3 && ii == 1;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (i < NI) {
+              if constexpr (RATIO) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[j][k], a[p][k], acc[i][j], 0, 0, 0);
+              } else if (k == 1) {
+                v4f t = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[j][0], a[p][0], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[j][1], a[p][1], t, 0, 0, 0);
+                asm volatile("" : "+v"(t)::"memory");
+                __builtin_amdgcn_sched_barrier(0);
+                const float s = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sc), kb));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[i][j][e] += t[e] * s;
+              }
+              asm volatile("" : "+v"(acc[i][j])::"memory");
+            }
+            if constexpr (RATIO) {
+              const int mj = 2 * k + (j >> 1), me = 2 * (j & 1);
+              if (mul_next) {
+                acc[(i + 1) % NI][mj][me] *= r;
+                acc[(i + 1) % NI][mj][me + 1] *= r;
+              }
+              if (mul_first) {
+                acc[0][mj][me] *= r1;
+                acc[0][mj][me + 1] *= r1;
+              }
+            }
+            if (ih == 1 && ii == 3 && k == 1) b[j][0] = fp8x8_to_f16x8((uint32_t)raw[j][0], (uint32_t)raw[j][1]);
+            if (ih == 0 && ii == 0 && k == 0) b[j][1] = fp8x8_to_f16x8((uint32_t)raw[j][2], (uint32_t)raw[j][3]);
+          }
+        }
+        // direct loads, one after each row fragment
+        if (ii == 0) {
+          const uint32_t so = (uint32_t)(ih * 128 + 16 * x.w) * (I * 2) + ka * 256 + h * 128;
+          bdma16(ra, x.va, so, x.l0 + ls * W_AREG + x.w * 2048);
+        }
+        if (ii == 1) {
+          const uint32_t so = (uint32_t)(ih * 128 + 16 * x.w) * (I * 2) + ka * 256 + h * 128;
+          bdma16(ra, w_va1(x), so, x.l0 + ls * W_AREG + x.w * 2048 + 1024);
+        }
+        if (h == 1 && ii >= 2) {
+          const uint32_t so = (uint32_t)(2 * x.w + ih) * 16 * I + kbb * BLK;
+          bdma16(rb, ii == 2 ? x.vb : w_vb1(x), so, x.l0 + W_B_OFF + (kb & 1) * W_BSLOT + (2 * x.w + ih) * 2048 + (ii - 2) * 1024);
+        }
+        if (q == 0 && ii == 2 && kb == NB_I - 2) w_load_meta(x, nxt, st.buf ^ 1);
+      }
+      if (q == 1) wait_vmcnt<4>();
+      else if (q == 3) wait_vmcnt<8>();
+      else wait_vmcnt<6>();
+      lds_barrier();
+      st.aslot = ns;
+    }
+  }
+}
+
+// An item: its scales' ratios, the K loop, and its rows, times the pairs' routing weights.
+template <int NI>
+__device__ __forceinline__ void w_one(const WCtx& x, const WItem& it, const WSrc& cur, const WSrc& nxt, WState& st) {
+  const int lane = opaque(x.lane), sl = lane & 15;
+  // scale of K block lane % 16 of this wave's 128-column block, with the 2^8 of C
+  const float sc = *reinterpret_cast<const float*>(x.lds + W_S_OFF + st.buf * 256 + (x.wn >> 1) * 64 + sl * 4) * C_LOAD_SCALE;
+  const float prev = __shfl(sc, (lane & 48) | ((sl + 15) & 15));
+  const float ratio = sl == 0 ? 1.0f : prev / sc;
+  float mx = fabsf(sc), mn = mx;
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, d));
+    mn = fminf(mn, __shfl_xor(mn, d));
+  }
+  // (fmaxf and fminf drop NaNs: every lane's own scale is tested)
+  const bool ok = fabsf(sc) > 1.0e-25f && fabsf(sc) < 1.0e25f && mx * 9.0e-13f < mn;
+  const bool ratio_ok = __builtin_amdgcn_ballot_w64(!ok) == 0;
+  v4f acc[NI][4];
+  v8h b[4][2], a[2][2];
+  v4i raw[4];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  const uint8_t* bs = x.lds + W_B_OFF + (4 * x.wn) * 2048;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    raw[j] = *reinterpret_cast<const v4i*>(bs + j * 2048 + x.flo);
+    b[j][0] = fp8x8_to_f16x8((uint32_t)raw[j][0], (uint32_t)raw[j][1]);
+  }
+  const uint8_t* as = x.lds + st.aslot * W_AREG + x.wm * 2048;
+  a[0][0] = *reinterpret_cast<const v8h*>(as + x.flo);
+  a[0][1] = *reinterpret_cast<const v8h*>(as + x.fhi);
+  float fin;
+  if (ratio_ok) {
+    w_run<NI, true>(x, it, cur, nxt, st, ratio, sc, acc, b, raw, a);
+    fin = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sc), NB_I - 1)) * C_STORE_SCALE;
+  } else {
+    w_run<NI, false>(x, it, cur, nxt, st, ratio, sc, acc, b, raw, a);
+    fin = C_STORE_SCALE;
+  }
+  const int el = opaque(x.lane), fr = el & 15, kg = el >> 4;
+  // lane (fr, kg) holds, of token row 16 (2 i + wm) + fr, columns 16 j + 4 kg + [0, 4): a 4 x 4
+  // transposition over the lane groups kg gives it columns 16 kg + [0, 16), two 16 B stores
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = 16 * (2 * i + x.wm) + fr;
+    const float w = *reinterpret_cast<const float*>(x.lds + W_PW_OFF + st.buf * (W_BM * 4) + row * 4) * fin;
+    uint32_t v[4][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        v[j][p] = f16x2_sat(acc[i][j][2 * p] * w, acc[i][j][2 * p + 1] * w);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const auto t = __builtin_amdgcn_permlane32_swap(v[j][p], v[j + 2][p], false, false);
+        v[j][p] = t[0];
+        v[j + 2][p] = t[1];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const auto t = __builtin_amdgcn_permlane16_swap(v[j][p], v[j + 1][p], false, false);
+        v[j][p] = t[0];
+        v[j + 1][p] = t[1];
+      }
+    }
+    if (row < it.valid) {
+      v4i* dst = reinterpret_cast<v4i*>(x.partial + (size_t)(it.seg + it.m0 + row) * H + it.nt * W_BN + x.wn * 64 + 16 * kg);
+      dst[0] = v4i{(int)v[0][0], (int)v[0][1], (int)v[1][0], (int)v[1][1]};
+      dst[1] = v4i{(int)v[2][0], (int)v[2][1], (int)v[3][0], (int)v[3][1]};
+    }
+  }
+  st.buf ^= 1;
+}
+
+__global__ __launch_bounds__(W_THREADS, 1) void gemm2_wide_kernel(
+    const uint16_t* __restrict__ c_act, const uint8_t* __restrict__ w2, const float* __restrict__ s2,
+    const DispatchHeader* __restrict__ hdr, const float* __restrict__ perm_w, uint16_t* __restrict__ partial) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t w_lds[];
+  __shared__ TileMap map;
+  const int tid = threadIdx.x, lane = tid & 63;
+  build_tile_map<W_BM>(hdr, map);
+  WCtx x;
+  x.c_act = c_act; x.w2 = w2; x.s2 = s2; x.perm_w = perm_w; x.partial = partial; x.lds = w_lds;
+  x.l0 = lds_addr(w_lds);
+  x.w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  x.lane = lane;
+  x.wm = x.w & 1; x.wn = x.w >> 1;
+  frag_sw_offsets(lane, x.flo, x.fhi);
+  const int rr = lane >> 3, p = (lane & 7) ^ rr;
+  x.va = (uint32_t)(rr * (I * 2) + p * 16);
+  // W2's 16 B chunk 4 h + g (K half h, lane group g) sits at position 2 g + h
+  x.vb = (uint32_t)(rr * I + (4 * (p & 1) + (p >> 1)) * 16);
+  const int total = __builtin_amdgcn_readfirstlane(map.total_m) * W_NT, G = gridDim.x;
+  const int slot = xcd_remap(blockIdx.x, G);
+  WItem it, nit;
+  if (!w_item(map, 0, slot, G, total, it)) return;
+  WState st{0, 0};
+  WSrc cur = w_src(x, it, true);
+  w_load_meta(x, cur, 0);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) w_load_a(x, cur.a, 0, u, u);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) w_load_b(x, cur.b, u >> 1, u & 1, u >> 1);
+  wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll 1
+  for (int r = 1;; ++r) {
+    const bool have = w_item(map, r, slot, G, total, nit);
+    if (!have) nit = it;
+    const WSrc nxt = w_src(x, nit, have);
+    const int nf = (it.valid + 15) / 16, ni = (nf - x.wm + 1) / 2;
+    if (ni > 6) w_one<8>(x, it, cur, nxt, st);
+    else if (ni > 4) w_one<6>(x, it, cur, nxt, st);
+    else if (ni > 2) w_one<4>(x, it, cur, nxt, st);
+    else w_one<2>(x, it, cur, nxt, st);
+    if (!have) break;
+    it = nit;
+    cur = nxt;
+  }
+  wait_vmcnt<0>();
+}
+
+// ---------------------------------------------------------------------------
 // Ordered combine: out[t] = bf16( sum_j pair row(t, j) ) over t's local experts
 // in ascending id, the rows decoded from fp16 (x 2^8, exact) and summed in fp32;
 // zeros for tokens with none. Each lane takes 8 columns, one 16 B load per pair.
@@ -1752,6 +2102,18 @@ hipError_t launch_gemm2_loader(const uint16_t* c_act, const uint8_t* w2, const f
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(gemm2_loader_kernel, dim3(grid), dim3(W2_THREADS), 2 * W2_STAGE, stream, c_act, w2, s2, hdr,
                      perm_w, partial);
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm2_wide(const uint16_t* c_act, const uint8_t* w2, const float* s2, const DispatchHeader* hdr,
+                             const float* perm_w, uint16_t* partial, int grid, hipStream_t stream) {
+  static PerDeviceOnce<hipError_t> once;
+  hipError_t e = hipErrorInvalidDevice;
+  once.get([] { return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm2_wide_kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, W_LDS); },
+           e);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(gemm2_wide_kernel, dim3(grid), dim3(W_THREADS), W_LDS, stream, c_act, w2, s2, hdr, perm_w, partial);
   return hipGetLastError();
 }
 

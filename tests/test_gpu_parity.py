@@ -452,6 +452,34 @@ def test_gemm2_item_heights_match_oracle(weights, dev, counts):
     assert_close_bf16(out, ref, f"counts={counts}")
 
 
+# W2 block scales for the wide GEMM2 (from 3,000 tokens): as made; one K block's scales 0 and one negative;
+# scales that differ by 2^44 within a row (both outside what its rescaled accumulators take).
+@pytest.mark.parametrize("scales", ["usual", "zero-negative", "far-apart"])
+def test_wide_gemm2_row_counts_and_scales_match_oracle(weights, dev, scales):
+    """At 3,000 tokens and more GEMM2 takes 256-row items: experts with row counts at
+    the edges of its fragments, steps and tiles, with usual block scales and with
+    scales that take its general path, against the oracle."""
+    counts = EDGE_COUNTS + [511, 513, 3, 240]
+    offset = 32
+    lg, b = _routing_for_counts(counts, offset, 4949)
+    T = lg.shape[0]
+    assert T >= 3000
+    _say(f"wide GEMM2 T={T} scales={scales}")
+    hs, hss = wl.quantize_1x128(wl.hidden_bf16(T, 4950).to(torch.float32))
+    cpu_w = list(weights[0])
+    s2 = cpu_w[3].clone()
+    if scales == "zero-negative":
+        s2[:, :, 3] = 0.0
+        s2[:, 1::2, 7] *= -1.0
+    elif scales == "far-apart":
+        s2[:, ::2, 5] *= 2.0 ** -44
+    cpu_w[3] = s2
+    gpu = [t.to(dev) for t in (lg, b, hs, hss)] + list(weights[1])[:3] + [s2.to(dev)]
+    out = fm.run(*gpu, offset, 2.5).float().cpu().numpy()
+    ref = cpu_ref.run(lg, b, hs, hss, *cpu_w, offset, 2.5).float().numpy()
+    assert_close_bf16(out, ref, f"wide GEMM2 scales={scales}")
+
+
 DECODE_EDGE_COUNTS = [[64], [33, 31], [17, 16, 15, 1, 0, 15], [1] * 32, [0] * 31 + [48], [2, 3, 4, 5, 6, 7, 8, 9],
                       [96], [65, 31], [3] * 32, [0] * 31 + [90], [30, 0, 31, 35]]
 
