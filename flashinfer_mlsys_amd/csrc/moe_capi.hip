@@ -45,7 +45,7 @@ constexpr int kMaxDevices = 64;
 constexpr int kDecodeMaxTokens = MOE_FP8_DECODE_MAX_TOKENS;  // decode shape (LDS dispatch, streaming GEMMs)
 static_assert(kDecodeMaxTokens <= moe::SMALL_T, "the decode kernels' LDS dispatch holds SMALL_T tokens");
 // Prefill GEMM2: 256-row items from here on (94 rows per expert when routing is even). GEMM2 alone, loader /
-// wide kernel, us: T=2000 129 / 137, 2,500 151 / 162, 3,001 173 / 169, 4,096 212 / 190.
+// wide kernel, us: T=768 83 / 98, 1,024 91 / 105, 2,000 129 / 137, 2,500 151 / 162, 3,001 173 / 169, 4,096 212 / 190.
 constexpr int kWideMinTokens = 3000;
 constexpr int kRouteInGemm1MaxTokens = 8;   // and routing inside GEMM1 (one token per wave) up to this many
 std::atomic<int> g_cu_count[kMaxDevices];

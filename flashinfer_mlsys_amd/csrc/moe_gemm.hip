@@ -1210,12 +1210,351 @@ __device__ __forceinline__ void p1_run_item(const P1Ctx& x, const P1Item& ic, co
   }
 }
 
+// ---------------------------------------------------------------------------
+// GEMM1 with few rows per expert ("thin" items).
+//
+// With at most 64 rows on (nearly) every expert GEMM1 is bound by reading the active
+// experts' weights once, and the tiled items' rounds decide its time: 19 active
+// experts are 304 items, two rounds of 256 workgroups for 1.2. Here
+//  * the work is split into groups of 8 column pairs and the workgroups of an expert
+//    divide its groups evenly, in sub-items of at most 16 groups;
+//  * a wave streams the weights of its (at most 2) groups straight into MFMA operand
+//    registers, 4 K blocks ahead, over the whole K: no reduction across waves, no
+//    weights in LDS. The activation rows, which all waves share, go through registers
+//    into two LDS slots, one barrier per K block;
+//  * all loads are buffer loads, unconditional (out of range: zeros, no traffic) and in
+//    the same order in every block, across sub-items too (the next sub-item's first
+//    blocks load during the last ones), so the compiler counts the loads in flight.
+// An expert with more than 64 rows is several "slices" of 64, each reading the weights
+// again; the kernel takes this path while that adds at most a quarter and the tiled
+// items' rounds waste more (the rule is in the kernel).
+//
+// Measured (GEMM1 alone, us, tiled -> thin; the weights' bytes at the thin rate): 11
+// active experts 70 -> 57 (5.7 TB/s), 17 134 -> 93 (5.4), 19 136 -> 100-106, 23 140 -> 129,
+// 24 143 -> 143; 32 165 -> 171. The same reads alone in a probe: 6.0 TB/s. (The same
+// structure for GEMM2 was 5-10 us faster than the loader kernel with 28-32 active
+// experts and as much slower with 23-27, whole calls; not kept.)
+// ---------------------------------------------------------------------------
+constexpr int TH_ROWS = 64;
+constexpr int TH_MAX = E_LOCAL + E_LOCAL / 4;
+struct ThinMap {
+  int e[TH_MAX], m0[TH_MAX];  // slice -> expert, first row
+  int cnt[E_LOCAL], seg[E_LOCAL];
+  int slices;                 // 0: too many rows for this path
+  int tiles;                  // 256-row tiles
+};
+
+__device__ __forceinline__ void build_thin_map(const DispatchHeader* hdr, ThinMap& m) {
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const int cnt = lane < E_LOCAL ? hdr->counts[lane] : 0;
+    const int n = (cnt + TH_ROWS - 1) / TH_ROWS;
+    int inc = n;
+#pragma unroll
+    for (int d = 1; d < E_LOCAL; d <<= 1) {
+      const int o = __shfl_up(inc, d);
+      if (lane >= d) inc += o;
+    }
+    const int total = __shfl(inc, E_LOCAL - 1);
+    const int act = __popcll(__ballot(cnt > 0));
+    const bool ok = total <= act + act / 4;
+    if (lane < E_LOCAL) {
+      m.cnt[lane] = cnt;
+      m.seg[lane] = hdr->seg_start[lane];
+      if (ok)
+        for (int k = 0; k < n; ++k) {
+          m.e[inc - n + k] = lane;
+          m.m0[inc - n + k] = k * TH_ROWS;
+        }
+    }
+    int tiles = (cnt + 255) / 256;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) tiles += __shfl_xor(tiles, d);
+    if (lane == 0) {
+      m.slices = ok ? total : 0;
+      m.tiles = tiles;
+    }
+  }
+  __syncthreads();
+}
+
+struct ThinItem {
+  int e, row0, valid, g0, size;  // row0: first pair row; groups g0 .. g0 + size - 1 of the expert
+};
+// A workgroup's range of column groups [pos, end) of one slice: slice s has the
+// workgroups from ceil(s G / n) to ceil((s + 1) G / n) - 1 (n slices, G workgroups), which
+// divide its GPE groups evenly. (One range over all slices' groups would be more
+// even still, but a range that crosses into the next expert costs a sub-item, and a
+// sub-item's K loop takes its latency however few its groups.)
+struct ThinRange {
+  int e, row0, valid, pos, end;
+};
+template <int GPE>
+__device__ __forceinline__ ThinRange thin_range(const ThinMap& m, int wg, int G) {
+  ThinRange r;
+  const int n = __builtin_amdgcn_readfirstlane(m.slices);
+  const int s = wg * n / G, first = (s * G + n - 1) / n, last = ((s + 1) * G + n - 1) / n;
+  r.pos = (wg - first) * GPE / (last - first);
+  r.end = (wg - first + 1) * GPE / (last - first);
+  r.e = __builtin_amdgcn_readfirstlane(m.e[s]);
+  const int m0 = __builtin_amdgcn_readfirstlane(m.m0[s]);
+  r.valid = min(TH_ROWS, __builtin_amdgcn_readfirstlane(m.cnt[r.e]) - m0);
+  r.row0 = __builtin_amdgcn_readfirstlane(m.seg[r.e]) + m0;
+  return r;
+}
+__device__ __forceinline__ bool thin_next(ThinRange& r, ThinItem& it) {
+  const int left = r.end - r.pos;
+  if (left <= 0) return false;
+  const int k = (left + 15) >> 4;
+  it.e = r.e;
+  it.row0 = r.row0;
+  it.valid = r.valid;
+  it.g0 = r.pos;
+  it.size = (left + k - 1) / k;
+  r.pos += it.size;
+  return true;
+}
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+constexpr uint32_t TH_NONE = 0xFFFFFF00u;  // an offset out of every resource's range
+
+// GEMM1 over thin items. Weight fragment of a group: W13 rows n..n+7 (X1) in lanes
+// 0-7 of each 16 and 2048+n.. (X2) in 8-15, as the decode GEMM1; it is the MFMA's first
+// operand, so lanes 0-31 hold X1 and 32-63 X2 of the same token and columns, brought
+// together by a swap of the lane halves between two row fragments.
+constexpr int T1_GPE = I / 8;               // 256 groups per expert
+constexpr int T1_A_BYTES = TH_ROWS * BLK;   // 8 KB: a K block of the rows
+constexpr int T1_SA_OFF = 2 * T1_A_BYTES;   // activation scales: 2 buffers of 8 blocks x 64 rows
+constexpr int T1_LDS = T1_SA_OFF + 2 * 8 * TH_ROWS * 4;
+static_assert(T1_LDS <= P1_LDS, "shares the tiled items' LDS");
+static_assert(NB_H % 8 == 0 && NB_I % 4 == 0, "the weight ring of 4 K blocks");
+
+struct T1Sub {
+  uint32_t w[2];       // this lane's weight offsets
+  float s1[2], s2[2];  // lane l: X1, X2 scale of K block l
+};
+
+struct T1Ctx {
+  __amdgpu_buffer_rsrc_t rw, ra, rs, rsw;
+  uint16_t* c_act;
+  uint8_t* lds;
+  int T, w, tid, flo, fhi;
+  uint32_t a, sa;  // this thread's activation row (tid / 8) and scale row (tid % 64)
+};
+
+// (No load here is waited for: that would drain the weights requested before it.)
+__device__ __forceinline__ void t1_sub(const T1Ctx& x, const ThinItem& it, bool have, T1Sub& s) {
+  const int tid = opaque(x.tid), lane = tid & 63, fr = lane & 15, kg = lane >> 4;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int j = 2 * x.w + k, g = it.g0 + j;
+    const bool on = have && j < it.size;
+    const int row = (fr < 8 ? fr : I + fr - 8) + 8 * g;
+    s.w[k] = on ? ((uint32_t)it.e * N1 + row) * H + kg * 32 : TH_NONE;
+    const uint32_t so = on && lane < NB_H ? ((uint32_t)(it.e * NB_N1 + g / 16) * NB_H + lane) * 4 : TH_NONE;
+    s.s1[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x.rsw, so, 0, 0));
+    s.s2[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x.rsw, so, NB_I * NB_H * 4, 0));
+  }
+}
+
+__device__ __forceinline__ v8i t1_load(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t so) {
+  const v4i lo = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, off, so, 0));
+  // (the 16 go into the scalar offset: a second vector offset would cost a register each)
+  const v4i hi = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, off, so + 16, 0));
+  return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
+struct T1Ring {
+  v8i w[4][2];  // weights of the next 4 K blocks
+  v4i a[4];     // activation bytes of blocks kb + 1 .. kb + 4 (loads complete in order: a shorter
+                // distance here would drain the weights requested before them)
+  float sa;     // activation scale for the next 8 blocks
+  int buf;      // scale buffer of the current 8 blocks (they are 7 to an item: runs on across items)
+};
+
+__device__ __forceinline__ v4i t1_load_a(const T1Ctx& x, uint32_t off, int kb) {
+  return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(x.ra, off, kb * BLK, 0));
+}
+__device__ __forceinline__ void t1_store_a(const T1Ctx& x, const v4i& a, int slot) {
+  const int r = x.tid >> 3;
+  *reinterpret_cast<v4i*>(x.lds + slot * T1_A_BYTES + (r >> 4) * FRAG_BYTES + frag_sw_offset(r & 15, x.tid & 7)) = a;
+}
+__device__ __forceinline__ void t1_store_sa(const T1Ctx& x, float sa, int buf) {
+  *reinterpret_cast<float*>(x.lds + T1_SA_OFF + (buf * 8 * TH_ROWS + x.tid) * 4) = sa;
+}
+// Scales of the 8 blocks from kb (row tid % 64, block kb + tid / 64).
+__device__ __forceinline__ float t1_load_sa(const T1Ctx& x, uint32_t sa, int kb) {
+  return __builtin_bit_cast(float,
+                            __builtin_amdgcn_raw_buffer_load_b32(x.rs, sa, (uint32_t)(kb + x.w) * x.T * 4, 0));
+}
+
+template <int NF>
+__device__ __forceinline__ void t1_run(const T1Ctx& x, const ThinItem& it, const T1Sub& cur, const T1Sub& nxt,
+                                       T1Ring& rg) {
+  const int lane = x.tid & 63;
+  v4f acc[NF][2];
+#pragma unroll
+  for (int i = 0; i < NF; ++i) acc[i][0] = acc[i][1] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int q = 0; q < NB_H / 8; ++q) {
+    const bool last = q == NB_H / 8 - 1;
+#pragma unroll
+    for (int jj = 0; jj < 8; ++jj) {
+      const int kb = 8 * q + jj, j = jj & 3;
+      lds_barrier();  // block kb's rows are in slot kb % 2; the other slot is read
+      t1_store_a(x, rg.a[(j + 1) & 3], (j + 1) & 1);
+      if (jj == 0) t1_store_sa(x, rg.sa, rg.buf ^ 1);
+      const bool na = last && jj >= 3;  // block kb + 5 is the next sub-item's (of the same rows)
+      __builtin_amdgcn_sched_barrier(0);
+      rg.a[(j + 1) & 3] = t1_load_a(x, x.a, na ? jj - 3 : kb + 5);
+      if (jj == 1) {
+        const int q2 = q + 2, q3 = q2 - NB_H / 8;
+        rg.sa = t1_load_sa(x, x.sa, 8 * (q3 < 0 ? q2 : q3));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      float sw[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cur.s1[k]), kb));
+        const float s2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cur.s2[k]), kb));
+        sw[k] = lane < 32 ? s1 : s2;
+      }
+      const uint8_t* as = x.lds + (j & 1) * T1_A_BYTES;
+      const float* sa = reinterpret_cast<const float*>(x.lds + T1_SA_OFF) + (rg.buf * 8 + jj) * TH_ROWS + (lane & 15);
+      v8i a[2];
+      float s[2];
+      a[0] = lds_frag_sw(as, x.flo, x.fhi);
+      s[0] = sa[0];
+#pragma unroll
+      for (int i = 0; i < NF; ++i) {  // (the next fragment is read ahead, one only: registers)
+        if (i + 1 < NF) {
+          a[(i + 1) & 1] = lds_frag_sw(as + (i + 1) * FRAG_BYTES, x.flo, x.fhi);
+          s[(i + 1) & 1] = sa[16 * (i + 1)];
+        }
+        v4f p[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) p[k] = mfma_fp8_k128(rg.w[j][k], a[i & 1]);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const float f = s[i & 1] * sw[k];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][k][r] += p[k][r] * f;
+          asm volatile("" : "+v"(acc[i][k]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const bool nw = last && jj >= 4;  // block kb + 4 is the next sub-item's
+#pragma unroll
+      for (int k = 0; k < 2; ++k) rg.w[j][k] = t1_load(x.rw, nw ? nxt.w[k] : cur.w[k], (nw ? jj - 4 : kb + 4) * BLK);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    rg.buf ^= 1;
+  }
+  // SwiGLU: row fragments i and i + 1 trade lane halves, then lanes 0-31 hold X1 and X2
+  // of fragment i, 32-63 of fragment i + 1: token row l % 16, columns 4 (l / 16 % 2) + r
+  const int el = opaque(x.tid) & 63;
+  const __amdgpu_buffer_rsrc_t rc = buf_rsrc(x.c_act + (size_t)it.row0 * I, (uint32_t)it.valid * I * 2);
+#pragma unroll
+  for (int i = 0; i < NF; i += 2)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      float x1[4], x2[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i][k][r]), __float_as_uint(acc[i + 1][k][r]),
+                                                        false, false);
+        x1[r] = __uint_as_float(t[0]);
+        x2[r] = __uint_as_float(t[1]);
+      }
+      const int row = 16 * (i + (el >> 5)) + (el & 15), j = 2 * x.w + k;
+      const uint32_t off = j < it.size ? (uint32_t)(row * I + 8 * (it.g0 + j) + 4 * ((el >> 4) & 1)) * 2 : TH_NONE;
+      const v2u v = {c_encode2(silu_mul(x1[0], x2[0]), silu_mul(x1[1], x2[1])),
+                     c_encode2(silu_mul(x1[2], x2[2]), silu_mul(x1[3], x2[3]))};
+      __builtin_amdgcn_raw_buffer_store_b64(v, rc, off, 0, 0);
+    }
+}
+
+// The workgroup's sub-items, with NF row fragments (its range is of one slice).
+template <int NF>
+__device__ __forceinline__ void t1_items(const T1Ctx& x, ThinRange& range, ThinItem it) {
+  ThinItem nit;
+  T1Sub cur, nxt;
+  t1_sub(x, it, true, cur);
+  T1Ring rg;
+  rg.buf = 0;
+  {
+    const v4i a0 = t1_load_a(x, x.a, 0);
+    const float sa0 = t1_load_sa(x, x.sa, 0);
+    rg.sa = t1_load_sa(x, x.sa, 8);
+#pragma unroll
+    for (int j = 1; j <= 4; ++j) rg.a[j & 3] = t1_load_a(x, x.a, j);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) rg.w[j][k] = t1_load(x.rw, cur.w[k], j * BLK);
+    t1_store_a(x, a0, 0);
+    t1_store_sa(x, sa0, 0);
+  }
+#pragma unroll 1
+  for (;;) {
+    const bool have = thin_next(range, nit);
+    if (!have) nit = it;
+    t1_sub(x, nit, have, nxt);
+    t1_run<NF>(x, it, cur, nxt, rg);
+    if (!have) break;
+    it = nit;
+    cur = nxt;
+  }
+}
+
+__device__ __forceinline__ void t1_body(const ThinMap& map, const uint8_t* hidden, const float* hscale, int T, int n_tok,
+                                        const uint8_t* w13, const float* s13, const int32_t* perm_tok, uint16_t* c_act,
+                                        uint8_t* lds) {
+  T1Ctx x;
+  x.rw = buf_rsrc(w13, (uint32_t)E_LOCAL * N1 * H);
+  x.ra = buf_rsrc(hidden, (uint32_t)n_tok * H);
+  x.rs = buf_rsrc(hscale, ((uint32_t)(NB_H - 1) * T + n_tok) * 4);
+  x.rsw = buf_rsrc(s13, (uint32_t)E_LOCAL * NB_N1 * NB_H * 4);
+  x.c_act = c_act; x.lds = lds; x.T = T;
+  x.tid = threadIdx.x;
+  x.w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  frag_sw_offsets(threadIdx.x & 63, x.flo, x.fhi);
+  ThinRange range = thin_range<T1_GPE>(map, xcd_remap(blockIdx.x, gridDim.x), gridDim.x);
+  ThinItem it;
+  if (!thin_next(range, it)) return;
+  {
+    const int tid = threadIdx.x, r = tid >> 3, rs = tid & (TH_ROWS - 1);
+    const __amdgpu_buffer_rsrc_t rt = buf_rsrc(perm_tok + it.row0, (uint32_t)it.valid * 4);
+    const uint32_t ta = __builtin_amdgcn_raw_buffer_load_b32(rt, r * 4, 0, 0);
+    const uint32_t ts = __builtin_amdgcn_raw_buffer_load_b32(rt, rs * 4, 0, 0);
+    x.a = r < it.valid ? ta * H + (tid & 7) * 16 : TH_NONE;
+    x.sa = rs < it.valid ? ts * 4 : TH_NONE;
+  }
+  if (it.valid <= 32) t1_items<2>(x, range, it);
+  else t1_items<4>(x, range, it);
+}
+
 __global__ __launch_bounds__(P1_THREADS, 1) void gemm1_prefill_kernel(
     const uint8_t* __restrict__ hidden, const float* __restrict__ hscale, int T, int n_tok, const uint8_t* __restrict__ w13,
     const float* __restrict__ s13, const DispatchHeader* __restrict__ hdr, const int32_t* __restrict__ perm_tok,
     uint16_t* __restrict__ c_act) {
   extern __shared__ __attribute__((aligned(16))) uint8_t p1_lds[];
-  __shared__ TileMap map;
+  __shared__ union {
+    TileMap tile;
+    ThinMap thin;
+  } maps;
+  build_thin_map(hdr, maps.thin);
+  const int slices = __builtin_amdgcn_readfirstlane(maps.thin.slices);  // uniform over the grid
+  // thin items where their reads come to less than three quarters of the tiled items'
+  // rounds, or nine tenths of an only round (GEMM1 us, tiled / thin, by slices: one round
+  // 11 70 / 57, 15 80.6 / 79.9; two 19 136 / 105, 23 140 / 129, 24 143 / 143, 26 148 / 153)
+  const int G = gridDim.x, tiled = __builtin_amdgcn_readfirstlane(maps.thin.tiles) * P1_NT, rounds = (tiled + G - 1) / G;
+  if (slices > 0 && (rounds == 1 ? 10 * P1_NT * slices < 9 * G : 4 * P1_NT * slices < 3 * rounds * G)) {
+    t1_body(maps.thin, hidden, hscale, T, n_tok, w13, s13, perm_tok, c_act, p1_lds);
+    return;
+  }
+  __syncthreads();
+  TileMap& map = maps.tile;
   const int tid = threadIdx.x, lane = tid & 63;
   build_tile_map<P1_BM>(hdr, map);
   P1Ctx x;
@@ -1224,7 +1563,7 @@ __global__ __launch_bounds__(P1_THREADS, 1) void gemm1_prefill_kernel(
   x.lane = lane;
   x.wm = x.w & 3; x.wn = x.w >> 2;
   frag_sw_offsets(lane, x.flo, x.fhi);
-  const int total = __builtin_amdgcn_readfirstlane(map.total_m) * P1_NT, G = gridDim.x;
+  const int total = __builtin_amdgcn_readfirstlane(map.total_m) * P1_NT;
   const int slot = xcd_remap(blockIdx.x, G);
   const bool one_tile = __builtin_amdgcn_ballot_w64((lane < E_LOCAL ? map.cnt[lane] : 0) > P1_BM) == 0;  // uniform
   P1Src ps;

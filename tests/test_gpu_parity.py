@@ -480,6 +480,28 @@ def test_wide_gemm2_row_counts_and_scales_match_oracle(weights, dev, scales):
     assert_close_bf16(out, ref, f"wide GEMM2 scales={scales}")
 
 
+THIN_COUNTS = {"one-round-split-expert": [65, 64, 40, 33, 32, 1, 0, 17], "two-rounds": [7] * 19,
+               "two-rounds-split-experts": [66, 127, 64] + [5, 0, 33] * 8 + [1] * 4, "just-tiled": [6] * 24}
+
+
+@pytest.mark.parametrize("name", list(THIN_COUNTS))
+def test_thin_gemm1_items_match_oracle(weights, dev, name):
+    """The prefill GEMM1 streams the weights (thin items) when few experts are active
+    and nearly all have at most 64 rows: experts of 1 to 64 rows and of 65 to 127 (two
+    slices), one and two rounds of the tiled items, and 24 experts, which it leaves to
+    the tiled items, against the oracle."""
+    counts, offset = THIN_COUNTS[name], 96
+    lg, b = _routing_for_counts(counts, offset, 7171 + sum(counts))
+    T = lg.shape[0]
+    assert T > 96
+    _say(f"thin GEMM1 T={T} {name}")
+    hs, hss = wl.quantize_1x128(wl.hidden_bf16(T, 7272 + T).to(torch.float32))
+    gpu = [t.to(dev) for t in (lg, b, hs, hss)] + list(weights[1])
+    out = fm.run(*gpu, offset, 2.5).float().cpu().numpy()
+    ref = cpu_ref.run(lg, b, hs, hss, *weights[0], offset, 2.5).float().numpy()
+    assert_close_bf16(out, ref, f"thin GEMM1 {name}")
+
+
 DECODE_EDGE_COUNTS = [[64], [33, 31], [17, 16, 15, 1, 0, 15], [1] * 32, [0] * 31 + [48], [2, 3, 4, 5, 6, 7, 8, 9],
                       [96], [65, 31], [3] * 32, [0] * 31 + [90], [30, 0, 31, 35]]
 
