@@ -284,8 +284,8 @@ def router_logits(hidden_bf16, gate_weight, out=None):
 
 @torch.no_grad()
 def router_logits_and_quantize(hidden_bf16, gate_weight, out=None):
-    """The producer side (one pass over the bf16 hidden states below 576 tokens,
-    the router and quantiser kernels in turn from 576 on): returns
+    """The producer side (one kernel, except for 2,049 to 2,303 tokens, where the router
+    and quantiser kernels run in turn): returns
     (routing_logits fp32 [T, 256], hidden_states e4m3 [T, 7168], hidden_states_scale
     fp32 [56, T]), bit for bit what ``router_logits`` and ``quantize_activations``
     return (reference moe/weight_origins_dataflow.md:19-21, :151-154). ``out`` may

@@ -48,7 +48,8 @@ __global__ __launch_bounds__(256) void quantize_1x128_kernel(const uint16_t* __r
     for (int k = 1; k < 16; k <<= 1) m = fmaxf(m, __shfl_xor(m, k));
     const float s = qblock_scale(m);
     if (valid) {
-      const uint32_t p0 = qblock_pack4(v[0], v[1], v[2], v[3], s), p1 = qblock_pack4(v[4], v[5], v[6], v[7], s);
+      const QDiv d = qblock_div(s);
+      const uint32_t p0 = qblock_pack4(v[0], v[1], v[2], v[3], d), p1 = qblock_pack4(v[4], v[5], v[6], v[7], d);
       *reinterpret_cast<uint2*>(qr + kb * BLK) = uint2{p0, p1};
       if (r == 0) scale[(size_t)kb * T + t] = s;
     }

@@ -10,15 +10,13 @@
 // then the 8 partial tiles are added through LDS in wave order (deterministic, no
 // atomics, no workspace).
 //
-// With QUANT the small-T kernel also writes the operator's FP8 activation inputs
-// (e4m3 rows [T, 7168] and 1 x 128 block scales [56, T]) from the hidden states
-// it reads anyway, with the quantiser kernel's arithmetic, each (token, K block)
-// exactly once: the workgroup of expert tile y quantises the K blocks kb with
-// kb % 16 == y from the fragments it holds (one pass over x instead of two:
-// 15 us instead of 20 at T=64). From RT2_MIN_T tokens on the two producer steps
-// run as the tiled kernel and the quantiser kernel: the same quantisation inside
-// the tiled kernel's compute waves (2 per SIMD, next to the loader waves) cost
-// more than the separate quantiser (84 against 49 + 40 us at T=8192).
+// With QUANT the kernels also write the operator's FP8 activation inputs (e4m3 rows [T,
+// 7168] and 1 x 128 block scales [56, T]) from the hidden states they read anyway, with
+// the quantiser kernel's arithmetic, each (token, K block) exactly once. In the small-T
+// kernel the workgroup of expert tile y quantises the K blocks kb with kb % 16 == y from
+// the fragments it holds (one pass over x instead of two: 15 us instead of 20 at T=64).
+// In the tiled kernels 4 more waves do it beside the GEMM (see rq_run; the same work in the
+// GEMM's compute waves took 84 us at T=8192, against 49 + 40 for the two kernels).
 //
 // Larger T: LDS-staged tiles of 128 tokens x 64 experts, 8 compute waves of
 // 32 x 32 (v_mfma_f32_32x32x16_bf16) and 4 loader waves that stream each 128-wide
@@ -93,11 +91,12 @@ __global__ __launch_bounds__(64 * RS_WAVES) void router_small_kernel(const uint1
       m = fmaxf(m, __shfl_xor(m, 16));
       m = fmaxf(m, __shfl_xor(m, 32));
       const float sc = qblock_scale(m);
+      const QDiv dv = qblock_div(sc);
       if (t < T) {
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
-          const uint32_t p0 = qblock_pack4(v[s4][0], v[s4][1], v[s4][2], v[s4][3], sc);
-          const uint32_t p1 = qblock_pack4(v[s4][4], v[s4][5], v[s4][6], v[s4][7], sc);
+          const uint32_t p0 = qblock_pack4(v[s4][0], v[s4][1], v[s4][2], v[s4][3], dv);
+          const uint32_t p1 = qblock_pack4(v[s4][4], v[s4][5], v[s4][6], v[s4][7], dv);
           *reinterpret_cast<uint2*>(q + (size_t)t * H + kb * BLK + 32 * s4 + 8 * kg) = uint2{p0, p1};
         }
         if (kg == 0) qs[(size_t)kb * T + t] = sc;
@@ -115,6 +114,119 @@ __global__ __launch_bounds__(64 * RS_WAVES) void router_small_kernel(const uint1
   }
 }
 
+// Quantiser waves of the tiled kernels (QUANT): 4 more waves a workgroup quantise its
+// items' tokens while the others run the GEMM, the workgroup of expert tile nt the K
+// blocks 14 nt .. 14 nt + 13 of them, so each (token, block) once. They take every
+// barrier of the K loop (a barrier counts all of a workgroup's waves) and do an equal
+// share of the item between two of them, their loads RQ_D steps ahead; x comes from
+// the caches, where the GEMM's own loads of the same rows bring it. A unit is 4 tokens
+// x 1 block: 16 lanes per token, 8 values (16 B) per lane. What bounds them is their
+// vector instructions between two barriers (with a division per value a K block took
+// 1.3 us instead of the GEMM's 0.6), hence the 3-instruction quotients and the paths of
+// finite blocks.
+constexpr int RQ_WAVES = 4, RQ_D = 4;
+constexpr int RQ_KB = NB_H / (E_GLOBAL / 64);  // 14 blocks per expert tile
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+struct RQuant {
+  __amdgpu_buffer_rsrc_t rx, rq, rs;
+  int T, lane, p;  // p: quantiser wave
+};
+__device__ __forceinline__ RQuant rq_make(const uint16_t* x, int T, uint8_t* q, float* qs, int p) {
+  RQuant r;
+  r.rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), (short)0, (int)((uint32_t)T * (H * 2)), 0x00020000);
+  r.rq = __builtin_amdgcn_make_buffer_rsrc(q, (short)0, (int)((uint32_t)T * H), 0x00020000);
+  r.rs = __builtin_amdgcn_make_buffer_rsrc(qs, (short)0, (int)((uint32_t)T * (NB_H * 4)), 0x00020000);
+  r.T = T; r.lane = threadIdx.x & 63; r.p = p;
+  return r;
+}
+// Units of token groups tg .. tg + NU - 1 from this lane's token t0, block kb. Rows at or past T
+// are out of the resources' ranges: zeros read, nothing written.
+template <int NU>
+__device__ __forceinline__ void rq_load(const RQuant& r, int t0, int tg, int kb, v4i (&raw)[NU]) {
+#pragma unroll
+  for (int n = 0; n < NU; ++n)
+    raw[n] = __builtin_bit_cast(
+        v4i, __builtin_amdgcn_raw_buffer_load_b128(r.rx, (uint32_t)t0 * (H * 2) + (r.lane & 15) * 16,
+                                                   (tg + n) * 4 * H * 2 + kb * (BLK * 2), 0));
+}
+template <int NU>
+__device__ __forceinline__ void rq_store(const RQuant& r, int t0, int tg, int kb, const v4i (&raw)[NU]) {
+  float v[NU][8], s[NU];
+  uint32_t o[NU][2];
+  bool finite = true;
+#pragma unroll
+  for (int n = 0; n < NU; ++n) {
+    const uint32_t w[4] = {(uint32_t)raw[n][0], (uint32_t)raw[n][1], (uint32_t)raw[n][2], (uint32_t)raw[n][3]};
+    bf16x8_to_f32(w, v[n]);
+    const float m = __uint_as_float(row16_max_bf16(w) << 16);  // NaN if a value is
+    s[n] = qblock_scale_finite(m);
+    qblock_pack8_finite(w, v[n], QDiv{s[n], __builtin_amdgcn_rcpf(s[n])}, o[n]);
+    finite = finite && m < __builtin_inff();
+  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0)) {
+#pragma unroll
+    for (int n = 0; n < NU; ++n) {
+      float m = 0.f;  // (the maximum of the block skips NaNs)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[n][i]));
+#pragma unroll
+      for (int k = 1; k < 16; k <<= 1) m = fmaxf(m, __shfl_xor(m, k));
+      s[n] = qblock_scale(m);
+      const QDiv d = qblock_div(s[n]);
+      o[n][0] = qblock_pack4(v[n][0], v[n][1], v[n][2], v[n][3], d);
+      o[n][1] = qblock_pack4(v[n][4], v[n][5], v[n][6], v[n][7], d);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NU; ++n) {
+    __builtin_amdgcn_raw_buffer_store_b64(v2u{o[n][0], o[n][1]}, r.rq, (uint32_t)t0 * H + (r.lane & 15) * 8,
+                                          (tg + n) * 4 * H + kb * BLK, 0);
+    const int t = t0 + 4 * (tg + n);
+    const bool first = (r.lane & 15) == 0 && t < r.T;  // (t < T: a row of the transposed scales must not run on)
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[n]), r.rs, first ? (uint32_t)t * 4 : 0xF0000000u,
+                                          (uint32_t)kb * r.T * 4, 0);
+  }
+}
+// All items of a workgroup (first, first + gridDim.x, ...): at each of an item's first STEPS K
+// blocks NU units a wave, token groups NU (k % TGS) .. of block k / TGS; EXTRA more
+// barriers after each item's last K block.
+template <int BM, int NU, int EXTRA>
+__device__ __forceinline__ void rq_run(const RQuant& r, int first, int n_items) {
+  constexpr int NT = E_GLOBAL / 64, TG = BM / 4 / RQ_WAVES, TGS = TG / NU, STEPS = TGS * RQ_KB;
+  static_assert(TG % NU == 0 && STEPS <= NB_H && STEPS % RQ_D == 0 && NB_H % RQ_D == 0 && RQ_D % TGS == 0, "steps");
+  auto token = [&](int i) {  // this lane's first token in item i (past the end: out of range)
+    const int item = first + i * (int)gridDim.x;
+    return (i < n_items ? item / NT * BM : r.T) + 4 * r.p * TG + (r.lane >> 4);
+  };
+  auto block = [&](int i) { return (first + i * (int)gridDim.x) % NT * RQ_KB; };
+  v4i buf[RQ_D][NU];
+  int t0 = token(0), kb0 = block(0);
+#pragma unroll
+  for (int d = 0; d < RQ_D; ++d) rq_load<NU>(r, t0, d % TGS * NU, kb0 + d / TGS, buf[d]);
+#pragma unroll 1
+  for (int i = 0; i < n_items; ++i) {
+    const int t1 = token(i + 1), kb1 = block(i + 1);
+#pragma unroll 1
+    for (int k = 0; k < NB_H; k += RQ_D) {
+      const bool last = k + RQ_D >= STEPS;
+      const int tn = last ? t1 : t0, kn = last ? kb1 : kb0 + (k + RQ_D) / TGS;
+#pragma unroll
+      for (int d = 0; d < RQ_D; ++d) {
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (STEPS == NB_H || k < STEPS) {  // uniform
+          rq_store<NU>(r, t0, d % TGS * NU, kb0 + k / TGS + d / TGS, buf[d]);
+          rq_load<NU>(r, tn, d % TGS * NU, kn + d / TGS, buf[d]);
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EXTRA; ++e) __builtin_amdgcn_s_barrier();
+    t0 = t1;
+    kb0 = kb1;
+  }
+}
+
 constexpr int RT2_BM = 128;                                  // tokens per item
 constexpr int RT2_BN = 64;                                   // experts per item
 constexpr int RT2_NT = E_GLOBAL / RT2_BN;                    // 4 expert tiles
@@ -127,8 +239,10 @@ constexpr int RT2_JOBS = RT2_STAGE / 1024 / RT2_PWAVES;      // 12 load instruct
 constexpr int RT2_MIN_T = 576;
 static_assert(RT2_JOBS * RT2_PWAVES * 1024 == RT2_STAGE, "load split");
 
-__global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES), 1) void router_tiled_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ g, int T, float* __restrict__ logits) {
+template <bool QUANT>
+__global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES + (QUANT ? RQ_WAVES : 0)), 1) void router_tiled_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ g, int T, float* __restrict__ logits,
+    uint8_t* __restrict__ q, float* __restrict__ qs) {
   extern __shared__ __attribute__((aligned(16))) uint8_t rt_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -138,6 +252,10 @@ __global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES), 1) void router_tile
   for (int item = first; item < total; item += gridDim.x) ++n_items;
   const int G = n_items * NB_H;
 
+  if (QUANT && wave >= RT2_CWAVES + RT2_PWAVES) {
+    rq_run<RT2_BM, 2, 0>(rq_make(x, T, q, qs, wave - RT2_CWAVES - RT2_PWAVES), first, n_items);
+    return;
+  }
   if (wave >= RT2_CWAVES) {
     // loader wave p: jobs 12 p .. 12 p + 11 of the 48 per block (0-31 hidden rows,
     // 32-47 gate rows); a job moves 8 rows x 128 B (one line of a K block)
@@ -255,8 +373,10 @@ __device__ __forceinline__ void rt3_wait_blocks(int n) {
   }
 }
 
-__global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES), 1) void router_ksplit_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ g, int T, float* __restrict__ logits) {
+template <bool QUANT>
+__global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES + (QUANT ? RQ_WAVES : 0)), 1) void router_ksplit_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ g, int T, float* __restrict__ logits,
+    uint8_t* __restrict__ q, float* __restrict__ qs) {
   extern __shared__ __attribute__((aligned(16))) uint8_t rt_lds[];
   float* red = reinterpret_cast<float*>(rt_lds + RT3_NSTAGE * RT3_STAGE);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -267,6 +387,11 @@ __global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES), 1) void router_kspl
   for (int item = first; item < total; item += gridDim.x) ++n_items;
   const int G = n_items * NB_H;
 
+  if (QUANT && wave >= RT2_CWAVES + RT2_PWAVES) {
+    // (28 units a wave and item: one at each of the first 28 K blocks)
+    rq_run<RT3_BM, 1, 1>(rq_make(x, T, q, qs, wave - RT2_CWAVES - RT2_PWAVES), first, n_items);
+    return;
+  }
   if (wave >= RT2_CWAVES) {
     // loader wave p: jobs 6 p .. 6 p + 5 of the 24 per block (0-7 hidden rows,
     // 8-23 gate rows); a job moves 8 rows x 128 B (one line of a K block)
@@ -366,48 +491,71 @@ __global__ __launch_bounds__(64 * (RT2_CWAVES + RT2_PWAVES), 1) void router_kspl
 
 hipError_t launch_quantize_1x128(const uint16_t* x, int T, uint8_t* q, float* scale, hipStream_t stream);
 
-static hipError_t launch_router_tiled(const uint16_t* x, const uint16_t* g, int T, float* logits, int cu,
-                                      hipStream_t stream) {
+// Whether the quantiser waves pay from RT2_MIN_T tokens on: the tiled kernel's first few
+// token counts leave a quarter of the CUs busy, whose quantiser waves then take longer than
+// the quantiser kernel on all of them (both steps, us, in turn / together: T=1,024
+// 27.5 / 25.1, 2,048 32.2 / 26.2 | 2,049 45.2 / 46.8, 3,000 50.2 / 46.2, 4,100 68.0 / 60.3,
+// 8,192 93.9 / 74.4, 14,107 165 / 138).
+constexpr int RQ_MIN_TILED_T = 2304;
+static bool rq_fused(int T, int cu) {
+  return T >= RQ_MIN_TILED_T || (T + RT3_BM - 1) / RT3_BM * RT2_NT <= cu;
+}
+
+// (q, qs null: the logits alone)
+static hipError_t launch_router_tiled(const uint16_t* x, const uint16_t* g, int T, float* logits, uint8_t* q, float* qs,
+                                      int cu, hipStream_t stream) {
   static PerDeviceOnce<hipError_t> once;
   hipError_t e = hipErrorInvalidDevice;
-  once.get([] { return hipFuncSetAttribute(reinterpret_cast<const void*>(router_tiled_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, RT2_NSTAGE * RT2_STAGE); },
-           e);
+  once.get([] {
+    const hipError_t r = hipFuncSetAttribute(reinterpret_cast<const void*>(router_tiled_kernel<false>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, RT2_NSTAGE * RT2_STAGE);
+    return r != hipSuccess ? r
+                           : hipFuncSetAttribute(reinterpret_cast<const void*>(router_tiled_kernel<true>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, RT2_NSTAGE * RT2_STAGE);
+  }, e);
   if (e != hipSuccess) return e;
   const int items = (T + RT2_BM - 1) / RT2_BM * RT2_NT;
   const int grid = min((items + 7) / 8 * 8, (cu + 7) / 8 * 8);
-  hipLaunchKernelGGL(router_tiled_kernel, dim3(grid), dim3(64 * (RT2_CWAVES + RT2_PWAVES)), RT2_NSTAGE * RT2_STAGE,
-                     stream, x, g, T, logits);
+  const int threads = 64 * (RT2_CWAVES + RT2_PWAVES + (q ? RQ_WAVES : 0));
+  if (q) hipLaunchKernelGGL(router_tiled_kernel<true>, dim3(grid), dim3(threads), RT2_NSTAGE * RT2_STAGE, stream, x, g, T,
+                            logits, q, qs);
+  else hipLaunchKernelGGL(router_tiled_kernel<false>, dim3(grid), dim3(threads), RT2_NSTAGE * RT2_STAGE, stream, x, g, T,
+                          logits, q, qs);
   return hipGetLastError();
 }
 
-static hipError_t launch_router_ksplit(const uint16_t* x, const uint16_t* g, int T, float* logits, int cu,
-                                       hipStream_t stream) {
+static hipError_t launch_router_ksplit(const uint16_t* x, const uint16_t* g, int T, float* logits, uint8_t* q, float* qs,
+                                       int cu, hipStream_t stream) {
   static PerDeviceOnce<hipError_t> once;
   hipError_t e = hipErrorInvalidDevice;
-  once.get([] { return hipFuncSetAttribute(reinterpret_cast<const void*>(router_ksplit_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, RT3_LDS); },
-           e);
+  once.get([] {
+    const hipError_t r = hipFuncSetAttribute(reinterpret_cast<const void*>(router_ksplit_kernel<false>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, RT3_LDS);
+    return r != hipSuccess ? r
+                           : hipFuncSetAttribute(reinterpret_cast<const void*>(router_ksplit_kernel<true>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, RT3_LDS);
+  }, e);
   if (e != hipSuccess) return e;
   const int items = (T + RT3_BM - 1) / RT3_BM * RT2_NT;
   const int grid = min((items + 7) / 8 * 8, (cu + 7) / 8 * 8);
-  hipLaunchKernelGGL(router_ksplit_kernel, dim3(grid), dim3(64 * (RT2_CWAVES + RT2_PWAVES)), RT3_LDS, stream, x, g,
-                     T, logits);
+  const int threads = 64 * (RT2_CWAVES + RT2_PWAVES + (q ? RQ_WAVES : 0));
+  if (q) hipLaunchKernelGGL(router_ksplit_kernel<true>, dim3(grid), dim3(threads), RT3_LDS, stream, x, g, T, logits, q, qs);
+  else hipLaunchKernelGGL(router_ksplit_kernel<false>, dim3(grid), dim3(threads), RT3_LDS, stream, x, g, T, logits, q, qs);
   return hipGetLastError();
 }
 
 // the tiled GEMM by token count: 32-token items with the K steps split over the
 // waves while they fit on the CUs in one round, 128-token items beyond
-static hipError_t launch_router_gemm(const uint16_t* x, const uint16_t* g, int T, float* logits, int cu,
-                                     hipStream_t stream) {
-  return (T + RT3_BM - 1) / RT3_BM * RT2_NT <= cu ? launch_router_ksplit(x, g, T, logits, cu, stream)
-                                                  : launch_router_tiled(x, g, T, logits, cu, stream);
+static hipError_t launch_router_gemm(const uint16_t* x, const uint16_t* g, int T, float* logits, uint8_t* q, float* qs,
+                                     int cu, hipStream_t stream) {
+  return (T + RT3_BM - 1) / RT3_BM * RT2_NT <= cu ? launch_router_ksplit(x, g, T, logits, q, qs, cu, stream)
+                                                  : launch_router_tiled(x, g, T, logits, q, qs, cu, stream);
 }
 
 hipError_t launch_router_logits(const uint16_t* x, const uint16_t* g, int T, float* logits, int cu,
                                 hipStream_t stream) {
   if (T <= 0) return hipSuccess;
-  if (T >= RT2_MIN_T) return launch_router_gemm(x, g, T, logits, cu, stream);
+  if (T >= RT2_MIN_T) return launch_router_gemm(x, g, T, logits, nullptr, nullptr, cu, stream);
   hipLaunchKernelGGL(router_small_kernel<false>, dim3((T + RT_M - 1) / RT_M, E_GLOBAL / 16), dim3(64 * RS_WAVES), 0,
                      stream, x, g, T, logits, nullptr, nullptr);
   return hipGetLastError();
@@ -417,8 +565,11 @@ hipError_t launch_router_quantize(const uint16_t* x, const uint16_t* g, int T, f
                                   int cu, hipStream_t stream) {
   if (T <= 0) return hipSuccess;
   if (T >= RT2_MIN_T) {
-    const hipError_t e = launch_router_gemm(x, g, T, logits, cu, stream);
-    return e != hipSuccess ? e : launch_quantize_1x128(x, T, q, qs, stream);
+    if (!rq_fused(T, cu)) {
+      const hipError_t e = launch_router_gemm(x, g, T, logits, nullptr, nullptr, cu, stream);
+      return e != hipSuccess ? e : launch_quantize_1x128(x, T, q, qs, stream);
+    }
+    return launch_router_gemm(x, g, T, logits, q, qs, cu, stream);
   }
   hipLaunchKernelGGL(router_small_kernel<true>, dim3((T + RT_M - 1) / RT_M, E_GLOBAL / 16), dim3(64 * RS_WAVES), 0,
                      stream, x, g, T, logits, q, qs);

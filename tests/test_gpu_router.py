@@ -83,6 +83,25 @@ def test_fused_producer_equals_separate_kernels(dev, gate, T):
         assert torch.equal(q.cpu().view(torch.uint8), qr.view(torch.uint8)) and torch.equal(s.cpu(), sr)
 
 
+@pytest.mark.parametrize("T", [577, 2047, 2048, 2304, 2433, 8191, 17001])
+def test_quantiser_waves_equal_the_quantiser_kernel(dev, gate, T):
+    """The quantiser waves of the two tiled router kernels (whole and ragged token
+    tiles, one and several items per workgroup) against the router and quantiser kernels
+    alone, bit for bit, on values that leave the quick path too: zeros of both signs,
+    tiny blocks, infinities and NaNs."""
+    x = wl.hidden_bf16(T, 77).to(dev)
+    x[0, :128] = 0
+    x[1, 128:256] *= 1e-20
+    x[T // 2, 5:9] = torch.tensor([-0.0, 3e38, -3e38, 1e-39], dtype=torch.bfloat16, device=dev)
+    x[T - 1, 300] = float("inf")
+    x[T - 1, 7000] = float("nan")
+    lg, q, s = fm.router_logits_and_quantize(x, gate[1])
+    q1, s1 = fm.quantize_activations(x)
+    assert torch.equal(q.view(torch.uint8), q1.view(torch.uint8))
+    assert torch.equal(s.view(torch.int32), s1.view(torch.int32))
+    assert torch.equal(lg.view(torch.int32), fm.router_logits(x, gate[1]).view(torch.int32))
+
+
 @pytest.mark.parametrize("T", [37, 700])
 def test_producer_graph_replay(dev, gate, T):
     """The producer step (fused below 576 tokens, two kernels from 576) captured in a
