@@ -8,7 +8,7 @@
 //   then bf16 (ref_moe.py:164-168): in the decode shape inside GEMM2, in the
 //   prefill shape through one row per (token, expert) pair and the combine
 //
-// GEMM1 runs on the e4m3 MFMA (v_mfma_scale_f32_16x16x128_f8f6f4 with unit E8M0
+// GEMM1 runs on the e4m3 MFMA (v_mfma_f32_16x16x128_f8f6f4, the form without E8M0
 // scales). One MFMA covers exactly one 128-wide K block, so the fp32 block
 // scales are applied once per block: acc += P * (s_act[row, kb] * s_w[nb, kb]).
 // GEMM2 runs on the fp16 MFMA: e4m3 weights widen to fp16 exactly, and C is
@@ -26,12 +26,14 @@
 //   prefill   -- many rows per expert. Persistent workgroups walk a device-built
 //                list of (expert, row tile, column tile) items, moving operands
 //                global -> LDS with direct loads into a ring of stages, in the
-//                exact order the MFMA reads them. GEMM1 (gemm1_prefill_kernel):
-//                every wave computes and issues direct loads from inline asm.
-//                GEMM2 (gemm2_loader_kernel): loader waves issue the direct loads
-//                while compute waves run the MFMAs. The workgroups of one XCD take
+//                exact order the MFMA reads them. GEMM1 (gemm1_prefill_kernel) and,
+//                from 3,000 tokens, GEMM2 (gemm2_wide_kernel): every wave computes
+//                and issues direct loads from inline asm. GEMM2 below
+//                (gemm2_loader_kernel): loader waves move the operands while
+//                compute waves run the MFMAs. The workgroups of one XCD take
 //                consecutive items, which share operand tiles, so that XCD's L2
-//                serves the repeats.
+//                serves the repeats. With few active experts of few rows GEMM1
+//                streams the weights to registers instead (thin items).
 #include "moe_common.h"
 #include <type_traits>
 #include "moe_host.h"
@@ -1592,7 +1594,7 @@ __global__ __launch_bounds__(P1_THREADS, 1) void gemm1_prefill_kernel(
 // ---------------------------------------------------------------------------
 // GEMM2 (+ routing weight), prefill shape: 128 rows x 256 output columns per
 // item on the fp16 MFMA v_mfma_f32_32x32x16_f16 (full fp16 rate; the 16x16x32
-// form runs at well under half of it), 8 compute waves as 2 (rows) x 4
+// form was slower in this kernel's dependent chains), 8 compute waves as 2 (rows) x 4
 // (columns), each 64 x 64 = 2 x 2 tiles of 32 x 32 (row blocks 2 i + wm, so
 // the two row halves interleave), and 4 loader waves.
 //
@@ -1923,7 +1925,7 @@ __global__ __launch_bounds__(W2_THREADS, 1) void gemm2_loader_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// GEMM2 (+ routing weight), prefill shape from WIDE_MIN_TOKENS tokens: items of 256
+// GEMM2 (+ routing weight), prefill shape from 3,000 tokens: items of 256
 // rows x 256 output columns, 8 waves as 2 (rows) x 4 (columns), each 128 x 64 as 8 x 4
 // tiles of the fp16 16x16x32 MFMA (1.87 PFLOP/s on such data against 1.72 for the
 // 32x32x16 form: the card is power-limited, 2.05 against 1.80 GHz). The loader kernel's
