@@ -53,13 +53,6 @@ __device__ __forceinline__ v8i load_v8i(const uint8_t* p) {
   return r;
 }
 
-// silu(x2) * x1 in fp32 from the hardware's exp2 and reciprocal (1 ulp each): a few fp32
-// ulps, against the 2^-12 relative rounding of the fp16 result.
-__device__ __forceinline__ float silu_mul(float x1, float x2) {
-  constexpr float LOG2E = 1.44269504088896340736f;
-  return x2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x2 * -LOG2E)) * x1;
-}
-
 // Swizzled 16 x 128 B e4m3 fragment (2 KB), written by two direct loads of 8
 // whole row lines each: load j, lane l holds row 8 j + l / 8, 16 B chunk
 // (l % 8) ^ (l / 8) ^ j, at 1024 j + 16 l. An MFMA lane m (row m % 16, K bytes

@@ -130,6 +130,20 @@ def test_fast_sigmoid_error_bound():
     assert 0.0 < out.value <= 2.0 ** -20
 
 
+def test_swiglu_error_bound():
+    """The GEMM1 epilogues' SwiGLU against 64 bits: the exponential (2 units of 2^-24), the sum,
+    the division and the product (1 each) make 5."""
+    if not os.path.exists(TEST_SUPPORT_LIB):
+        raise FileNotFoundError(f"{TEST_SUPPORT_LIB} is not built (build() compiles it)")
+    lib = ctypes.CDLL(TEST_SUPPORT_LIB)
+    lib.moe_test_silu_max_relative_error.argtypes = [ctypes.POINTER(ctypes.c_double)]
+    lib.moe_test_silu_max_relative_error.restype = ctypes.c_int
+    out = ctypes.c_double(-1.0)
+    assert lib.moe_test_silu_max_relative_error(ctypes.byref(out)) == 0
+    _say(f"max relative error of silu_mul = {out.value * 2.0 ** 24:.2f} * 2^-24")
+    assert 0.0 < out.value <= 5 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("T,bias_kind", [(6144, "normal"), (6144, "tie"), (9000, "normal")])
 def test_route_fast_path_certification(dev, T, bias_kind):
     """From 6,144 tokens the routing kernel tries the fast scores first and keeps
