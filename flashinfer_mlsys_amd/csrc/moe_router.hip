@@ -140,14 +140,15 @@ __device__ __forceinline__ RQuant rq_make(const uint16_t* x, int T, uint8_t* q, 
   return r;
 }
 // Units of token groups tg .. tg + NU - 1 from this lane's token t0, block kb. Rows at or past T
-// are out of the resources' ranges: zeros read, nothing written.
+// are out of the resources' ranges: zeros read, nothing written. The row is all in the vector
+// offset, which alone decides the bounds check (the scalar offset stays inside a row).
 template <int NU>
 __device__ __forceinline__ void rq_load(const RQuant& r, int t0, int tg, int kb, v4i (&raw)[NU]) {
 #pragma unroll
   for (int n = 0; n < NU; ++n)
     raw[n] = __builtin_bit_cast(
-        v4i, __builtin_amdgcn_raw_buffer_load_b128(r.rx, (uint32_t)t0 * (H * 2) + (r.lane & 15) * 16,
-                                                   (tg + n) * 4 * H * 2 + kb * (BLK * 2), 0));
+        v4i, __builtin_amdgcn_raw_buffer_load_b128(r.rx, (uint32_t)(t0 + 4 * (tg + n)) * (H * 2) + (r.lane & 15) * 16,
+                                                   kb * (BLK * 2), 0));
 }
 template <int NU>
 __device__ __forceinline__ void rq_store(const RQuant& r, int t0, int tg, int kb, const v4i (&raw)[NU]) {
@@ -179,9 +180,8 @@ __device__ __forceinline__ void rq_store(const RQuant& r, int t0, int tg, int kb
   }
 #pragma unroll
   for (int n = 0; n < NU; ++n) {
-    __builtin_amdgcn_raw_buffer_store_b64(v2u{o[n][0], o[n][1]}, r.rq, (uint32_t)t0 * H + (r.lane & 15) * 8,
-                                          (tg + n) * 4 * H + kb * BLK, 0);
     const int t = t0 + 4 * (tg + n);
+    __builtin_amdgcn_raw_buffer_store_b64(v2u{o[n][0], o[n][1]}, r.rq, (uint32_t)t * H + (r.lane & 15) * 8, kb * BLK, 0);
     const bool first = (r.lane & 15) == 0 && t < r.T;  // (t < T: a row of the transposed scales must not run on)
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[n]), r.rs, first ? (uint32_t)t * 4 : 0xF0000000u,
                                           (uint32_t)kb * r.T * 4, 0);

@@ -102,6 +102,27 @@ def test_quantiser_waves_equal_the_quantiser_kernel(dev, gate, T):
     assert torch.equal(lg.view(torch.int32), fm.router_logits(x, gate[1]).view(torch.int32))
 
 
+@pytest.mark.parametrize("T", [577, 2305, 2433])
+def test_producer_writes_nothing_past_its_outputs(dev, gate, T):
+    """Ragged last token tiles: the outputs are the front of larger buffers (the rows of a
+    whole tile and more behind them), whose tails stay as they were. The hidden states are
+    the front of a larger buffer too, of NaNs behind the T rows."""
+    x = torch.full((T + 160, 7168), float("nan"), dtype=torch.bfloat16, device=dev)
+    x[:T] = wl.hidden_bf16(T, 78).to(dev)
+    sizes = {"logits": (T * 256 * 4, 160 * 256 * 4), "q": (T * 7168, 160 * 7168), "scale": (56 * T * 4, 56 * 160 * 4)}
+    buf = {k: torch.full((n + tail,), 0x5A, dtype=torch.uint8, device=dev) for k, (n, tail) in sizes.items()}
+    front = {k: buf[k][:sizes[k][0]] for k in buf}
+    out = (front["logits"].view(torch.float32).view(T, 256), front["q"].view(torch.float8_e4m3fn).view(T, 7168),
+           front["scale"].view(torch.float32).view(56, T))
+    print(f"producer guards T={T}", flush=True)
+    fm.router_logits_and_quantize(x[:T], gate[1], out=out)
+    for k, b in buf.items():
+        assert bool((b[sizes[k][0]:] == 0x5A).all()), k
+    q, s = fm.quantize_activations(x[:T])
+    assert torch.equal(out[1].view(torch.uint8), q.view(torch.uint8)) and torch.equal(out[2], s)
+    assert torch.equal(out[0], fm.router_logits(x[:T], gate[1]))
+
+
 @pytest.mark.parametrize("T", [37, 700])
 def test_producer_graph_replay(dev, gate, T):
     """The producer step (fused below 576 tokens, two kernels from 576) captured in a
