@@ -33,7 +33,7 @@ int gemm1_decode_blocks_per_cu(int T);
 hipError_t launch_gemm1_prefill(const uint8_t*, const float*, int, int, const uint8_t*, const float*,
                                const DispatchHeader*, const int32_t*, uint16_t*, int, hipStream_t);
 hipError_t launch_gemm2_loader(const uint16_t*, const uint8_t*, const float*, const DispatchHeader*, const float*,
-                               uint16_t*, int, hipStream_t);
+                               uint16_t*, bool, int, hipStream_t);
 hipError_t launch_gemm2_wide(const uint16_t*, const uint8_t*, const float*, const DispatchHeader*, const float*,
                              uint16_t*, int, hipStream_t);
 hipError_t launch_combine(const uint16_t*, const int32_t*, int, uint16_t*, hipStream_t);
@@ -44,9 +44,11 @@ namespace {
 constexpr int kMaxDevices = 64;
 constexpr int kDecodeMaxTokens = MOE_FP8_DECODE_MAX_TOKENS;  // decode shape (LDS dispatch, streaming GEMMs)
 static_assert(kDecodeMaxTokens <= moe::SMALL_T, "the decode kernels' LDS dispatch holds SMALL_T tokens");
-// Prefill GEMM2: 256-row items from here on (94 rows per expert when routing is even). GEMM2 alone, loader /
-// wide kernel, us: T=768 83 / 98, 1,024 91 / 105, 2,000 129 / 137, 2,500 151 / 162, 3,001 173 / 169, 4,096 212 / 190.
-constexpr int kWideMinTokens = 3000;
+// Prefill GEMM2: from here on the wide kernel (256-row items) and the loader kernel are both launched, and the
+// one that the experts' row counts favour does the work (moe_gemm.hip, g2_takes_wide). Whole calls with even
+// routing, us, loader kernel alone / both launched: T=3,200 388 / 393, 3,400 393 / 395 | 3,600 414 / 408, 4,096
+// 436 / 424, 8,192 712 / 671.
+constexpr int kWideMinTokens = 3500;
 constexpr int kRouteInGemm1MaxTokens = 8;   // and routing inside GEMM1 (one token per wave) up to this many
 std::atomic<int> g_cu_count[kMaxDevices];
 thread_local const char* t_last_hip_error = "no error";
@@ -187,8 +189,14 @@ hipError_t run_stage(int stage, const Call& c) {
                                  (cu_count() + 7) / 8 * 8, c.stream);
     case 2:
       if (c.decode) return launch_gemm2_decode(c.c_act, c.w2, c.s2, c.hdr, c.perm_tok, c.perm_w, c.T, c.out, c.stream);
-      return (c.T >= kWideMinTokens ? launch_gemm2_wide : launch_gemm2_loader)(
-          c.c_act, c.w2, c.s2, c.hdr, c.perm_w, c.partial, (cu_count() + 7) / 8 * 8, c.stream);
+      {
+        const int grid = (cu_count() + 7) / 8 * 8;
+        const bool wide = c.T >= kWideMinTokens;
+        hipError_t e = hipSuccess;
+        if (wide) e = launch_gemm2_wide(c.c_act, c.w2, c.s2, c.hdr, c.perm_w, c.partial, grid, c.stream);
+        if (e != hipSuccess) return e;
+        return launch_gemm2_loader(c.c_act, c.w2, c.s2, c.hdr, c.perm_w, c.partial, wide, grid, c.stream);
+      }
     case 3:
       if (c.decode) return hipSuccess;  // summed inside GEMM2
       return launch_combine(c.partial, c.tok_pair, c.T, c.out, c.stream);

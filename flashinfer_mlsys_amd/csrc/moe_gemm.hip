@@ -26,11 +26,12 @@
 //   prefill   -- many rows per expert. Persistent workgroups walk a device-built
 //                list of (expert, row tile, column tile) items, moving operands
 //                global -> LDS with direct loads into a ring of stages, in the
-//                exact order the MFMA reads them. GEMM1 (gemm1_prefill_kernel) and,
-//                from 3,000 tokens, GEMM2 (gemm2_wide_kernel): every wave computes
-//                and issues direct loads from inline asm. GEMM2 below
-//                (gemm2_loader_kernel): loader waves move the operands while
-//                compute waves run the MFMAs. The workgroups of one XCD take
+//                exact order the MFMA reads them. GEMM1 (gemm1_prefill_kernel) and
+//                GEMM2 of large calls with many rows per local expert
+//                (gemm2_wide_kernel): every wave computes and issues direct loads
+//                from inline asm. GEMM2 of the others (gemm2_loader_kernel): loader
+//                waves move the operands while compute waves run the MFMAs. The
+//                workgroups of one XCD take
 //                consecutive items, which share operand tiles, so that XCD's L2
 //                serves the repeats. With few active experts of few rows GEMM1
 //                streams the weights to registers instead (thin items).
@@ -1905,11 +1906,31 @@ __device__ __forceinline__ void g2_loader_body(const uint16_t* __restrict__ c_ac
   }
 }
 
+// Which of the two prefill GEMM2 kernels takes a call that is given to both (the wide
+// kernel's 256-row items, launched first, and this one's): the wide kernel from 75 rows per
+// 256-row tile of the local experts on. The token count does not tell: routing that
+// favours other ranks' experts leaves a call of many tokens with few local rows, whose
+// mostly empty wide items wait for W2. GEMM2 alone at T=4,096, loader / wide kernel, us, every expert
+// with 8 rows 95 / 116, 40 106 / 123, 64 113 / 129, 74 137 / 142, 86 140 / 146, 128 158 / 152; two
+// experts of 600 and 256 rows and the others with 30 136 / 137 (52 rows a tile), with 60 148 / 139 (78).
+// The kernel that leaves the call to the other one costs the call 2-3 us.
+constexpr int G2_WIDE_ROWS = 75;
+__device__ __forceinline__ bool g2_takes_wide(const DispatchHeader* hdr) {  // uniform over the grid
+  const int lane = threadIdx.x & 63;
+  const int cnt = lane < E_LOCAL ? hdr->counts[lane] : 0;
+  int d = cnt - G2_WIDE_ROWS * ((cnt + 255) / 256);
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) d += __shfl_xor(d, k);
+  return __builtin_amdgcn_readfirstlane(d) >= 0;
+}
+
 __global__ __launch_bounds__(W2_THREADS, 1) void gemm2_loader_kernel(
     const uint16_t* __restrict__ c_act, const uint8_t* __restrict__ w2, const float* __restrict__ s2,
-    const DispatchHeader* __restrict__ hdr, const float* __restrict__ perm_w, uint16_t* __restrict__ partial) {
+    const DispatchHeader* __restrict__ hdr, const float* __restrict__ perm_w, uint16_t* __restrict__ partial,
+    bool after_wide) {
   extern __shared__ __attribute__((aligned(16))) uint8_t q2_lds[];
   __shared__ TileMap map;
+  if (after_wide && g2_takes_wide(hdr)) return;
   // 64-row items when every expert has at most 64 rows (uniform over the grid)
   const int lane = threadIdx.x & 63;
   const bool small = __builtin_amdgcn_ballot_w64(lane < E_LOCAL && hdr->counts[min(lane, E_LOCAL - 1)] > Q2_BM / 2) == 0;
@@ -1918,7 +1939,7 @@ __global__ __launch_bounds__(W2_THREADS, 1) void gemm2_loader_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// GEMM2 (+ routing weight), prefill shape from 3,000 tokens: items of 256
+// GEMM2 (+ routing weight), large prefill calls (g2_takes_wide): items of 256
 // rows x 256 output columns, 8 waves as 2 (rows) x 4 (columns), each 128 x 64 as 8 x 4
 // tiles of the fp16 16x16x32 MFMA (1.87 PFLOP/s on such data against 1.72 for the
 // 32x32x16 form: the card is power-limited, 2.05 against 1.80 GHz). The loader kernel's
@@ -1951,9 +1972,9 @@ __global__ __launch_bounds__(W2_THREADS, 1) void gemm2_loader_kernel(
 // of fragment read are free of bank conflicts.
 //
 // Measured against the loader kernel (whole calls, us): skewed T=4096 1,500 -> 1,400,
-// T=14,107 1,086 -> 1,005, T=4096 451 -> 430, T=3001 389 -> 385; GEMM2 alone at T=2500
-// 151 -> 162, T=2000 129 -> 137, T=901 101 -> 126: most experts there have fewer than 100
-// rows, whose half-empty items cost more than the loader kernel's 64- and 128-row ones.
+// T=14,107 1,086 -> 1,005, T=4096 451 -> 430; GEMM2 alone at T=2500 151 -> 162, T=2000
+// 129 -> 137, T=901 101 -> 126: most experts there have fewer than 80 rows, whose
+// half-empty items cost more than the loader kernel's 64- and 128-row ones.
 // A block takes 5,650 clk on full items (4,608 of MFMAs).
 // ---------------------------------------------------------------------------
 constexpr int W_BM = 256, W_BN = 256;
@@ -2223,6 +2244,7 @@ __global__ __launch_bounds__(W_THREADS, 1) void gemm2_wide_kernel(
     const DispatchHeader* __restrict__ hdr, const float* __restrict__ perm_w, uint16_t* __restrict__ partial) {
   extern __shared__ __attribute__((aligned(16))) uint8_t w_lds[];
   __shared__ TileMap map;
+  if (!g2_takes_wide(hdr)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   build_tile_map<W_BM>(hdr, map);
   WCtx x;
@@ -2427,7 +2449,8 @@ hipError_t launch_gemm1_prefill(const uint8_t* hidden, const float* hscale, int 
 }
 
 hipError_t launch_gemm2_loader(const uint16_t* c_act, const uint8_t* w2, const float* s2, const DispatchHeader* hdr,
-                               const float* perm_w, uint16_t* partial, int grid, hipStream_t stream) {
+                               const float* perm_w, uint16_t* partial, bool after_wide, int grid,
+                               hipStream_t stream) {
   static PerDeviceOnce<hipError_t> once;
   hipError_t e = hipErrorInvalidDevice;
   once.get([] { return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm2_loader_kernel),
@@ -2435,7 +2458,7 @@ hipError_t launch_gemm2_loader(const uint16_t* c_act, const uint8_t* w2, const f
            e);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(gemm2_loader_kernel, dim3(grid), dim3(W2_THREADS), 2 * W2_STAGE, stream, c_act, w2, s2, hdr,
-                     perm_w, partial);
+                     perm_w, partial, after_wide);
   return hipGetLastError();
 }
 

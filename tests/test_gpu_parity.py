@@ -6,6 +6,7 @@ Everything goes through libmoe_mi355x.so's C ABI via flashinfer_mlsys_amd.
 """
 import ctypes
 import os
+import re
 
 import numpy as np
 import pytest
@@ -466,18 +467,65 @@ def test_gemm2_item_heights_match_oracle(weights, dev, counts):
     assert_close_bf16(out, ref, f"counts={counts}")
 
 
-# W2 block scales for the wide GEMM2 (from 3,000 tokens): as made; one K block's scales 0 and one negative;
+def _source_constant(file, name):
+    """An integer constant of the kernels' sources, so that a test of a rule follows it."""
+    path = os.path.join(os.path.dirname(fm.__file__), "csrc", file)
+    with open(path) as f:
+        found = re.findall(rf"constexpr int {name} = (\d+);", f.read())
+    assert len(found) == 1, f"{name} in {file}"
+    return int(found[0])
+
+
+def _takes_wide_gemm2(counts):
+    """The rule of g2_takes_wide (csrc/moe_gemm.hip) for a call that both GEMM2 kernels are given."""
+    tiles = sum((c + 255) // 256 for c in counts)
+    return sum(counts) >= _source_constant("moe_gemm.hip", "G2_WIDE_ROWS") * tiles
+
+
+@pytest.mark.parametrize("counts,wide", [([40] * 32, False), ([75] * 31 + [74], False), ([75] * 32, True),
+                                         ([0] * 20 + [600] + [5] * 11, False), ([0] * 20 + [600] + [50] * 11, True),
+                                         ([0] * 32, True)],
+                         ids=["cold", "below", "at", "one-hot-cold", "one-hot", "none"])
+def test_gemm2_kernel_follows_the_rows_per_expert(weights, dev, counts, wide):
+    """A call of 3,500 tokens or more whose routing favours other ranks' experts keeps the
+    loader GEMM2, which every call below runs: tokens are independent, so its output is
+    then bit for bit that of the same tokens in two smaller calls. With more rows per
+    256-row tile the wide kernel takes it, whose sums round differently."""
+    offset, line = 160, _source_constant("moe_capi.hip", "kWideMinTokens")
+    n = sum(counts)
+    lg, b = _routing_for_counts(counts, offset, 3535 + n) if n else (torch.empty((0, 256)), None)
+    T = line + 5
+    assert n <= T and wide == _takes_wide_gemm2(counts)
+    fill = torch.full((T - n, 256), -8.0)  # tokens of other ranks' experts
+    rng = np.random.default_rng(77)
+    for t in range(T - n):
+        for g, k in zip(rng.choice([g for g in range(8) if g != offset // 32], 4, replace=False), (2, 2, 2, 2)):
+            fill[t, g * 32 + torch.from_numpy(rng.choice(32, k, replace=False))] = 6.0 + float(rng.random())
+    lg = torch.cat([lg, fill])[torch.from_numpy(rng.permutation(T))].contiguous()
+    _say(f"GEMM2 kernel by rows: T={T} pairs={n} wide={wide}")
+    acts = [lg.to(dev), torch.zeros(256, dtype=torch.bfloat16, device=dev)]
+    hs, hss = (t.to(dev) for t in wl.quantize_1x128(wl.hidden_bf16(T, 3636).to(torch.float32)))
+    whole = fm.run(*acts, hs, hss, *weights[1], offset, 2.5)
+    half = T // 2
+    parts = torch.cat([fm.run(acts[0][a:z].contiguous(), acts[1], hs[a:z].contiguous(), hss[:, a:z].contiguous(),
+                              *weights[1], offset, 2.5) for a, z in ((0, half), (half, T))])
+    assert torch.equal(whole.view(torch.int16), parts.view(torch.int16)) == (not wide or n == 0)
+    err = (whole.float() - parts.float()).abs().max().item()
+    assert err <= ATOL + RTOL * parts.float().abs().max().item()
+
+
+# W2 block scales for the wide GEMM2 (from 3,500 tokens): as made; one K block's scales 0 and one negative;
 # scales that differ by 2^44 within a row (both outside what its rescaled accumulators take).
 @pytest.mark.parametrize("scales", ["usual", "zero-negative", "far-apart"])
 def test_wide_gemm2_row_counts_and_scales_match_oracle(weights, dev, scales):
-    """At 3,000 tokens and more GEMM2 takes 256-row items: experts with row counts at
+    """At 3,500 tokens and more GEMM2 takes 256-row items: experts with row counts at
     the edges of its fragments, steps and tiles, with usual block scales and with
     scales that take its general path, against the oracle."""
-    counts = EDGE_COUNTS + [511, 513, 3, 240]
+    counts = EDGE_COUNTS + [511, 513, 3, 240, 512]
     offset = 32
     lg, b = _routing_for_counts(counts, offset, 4949)
     T = lg.shape[0]
-    assert T >= 3000
+    assert T >= _source_constant("moe_capi.hip", "kWideMinTokens") and _takes_wide_gemm2(counts)
     _say(f"wide GEMM2 T={T} scales={scales}")
     hs, hss = wl.quantize_1x128(wl.hidden_bf16(T, 4950).to(torch.float32))
     cpu_w = list(weights[0])
