@@ -284,7 +284,7 @@ def router_logits(hidden_bf16, gate_weight, out=None):
 
 @torch.no_grad()
 def router_logits_and_quantize(hidden_bf16, gate_weight, out=None):
-    """The producer side (one kernel, except for 2,049 to 2,303 tokens, where the router
+    """The producer side (one kernel, except for 2,049 to 2,999 tokens, where the router
     and quantiser kernels run in turn): returns
     (routing_logits fp32 [T, 256], hidden_states e4m3 [T, 7168], hidden_states_scale
     fp32 [56, T]), bit for bit what ``router_logits`` and ``quantize_activations``

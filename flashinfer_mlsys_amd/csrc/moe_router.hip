@@ -493,10 +493,12 @@ hipError_t launch_quantize_1x128(const uint16_t* x, int T, uint8_t* q, float* sc
 
 // Whether the quantiser waves pay from RT2_MIN_T tokens on: the tiled kernel's first few
 // token counts leave a quarter of the CUs busy, whose quantiser waves then take longer than
-// the quantiser kernel on all of them (both steps, us, in turn / together: T=1,024
-// 27.5 / 25.1, 2,048 32.2 / 26.2 | 2,049 45.2 / 46.8, 3,000 50.2 / 46.2, 4,100 68.0 / 60.3,
-// 8,192 93.9 / 74.4, 14,107 165 / 138).
-constexpr int RQ_MIN_TILED_T = 2304;
+// the quantiser kernel on all of them. Both steps, us, in turn / together, calls back to back
+// on the same buffers: T=1,024 25.9 / 23.2, 2,048 29.0 / 25.6 | 2,049 42.8 / 46.6, 2,304
+// 43.2 / 46.4, 2,816 45.5 / 46.8 | 3,000 46.3 / 45.7, 4,100 51.1 / 48.4, 8,192 68.8 / 54.2,
+// 14,107 138 / 128 (one call with the caches full of other data: 2,304 68.3 / 74.4, 3,000
+// 73.4 / 69.9, 8,192 103 / 99).
+constexpr int RQ_MIN_TILED_T = 3000;
 static bool rq_fused(int T, int cu) {
   return T >= RQ_MIN_TILED_T || (T + RT3_BM - 1) / RT3_BM * RT2_NT <= cu;
 }

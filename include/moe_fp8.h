@@ -226,7 +226,7 @@ int moe_fp8_router_logits(const uint16_t* hidden_bf16, const uint16_t* gate_weig
  * Both producer-side steps (the router GEMM of moe_fp8_router_logits and the
  * quantiser of moe_fp8_quantize_activations, reference
  * moe/weight_origins_dataflow.md:19-21 and :21, :151-154, which read the same
- * x) in one kernel, except for 2,049 to 2,303 tokens (on 256 CUs), where the two
+ * x) in one kernel, except for 2,049 to 2,999 tokens (on 256 CUs), where the two
  * kernels run in turn; writes the same routing_logits, hidden_states and
  * hidden_states_scale, bit for bit, as the two separate calls. All pointers
  * 16-byte aligned. Stream-ordered.

@@ -1,4 +1,5 @@
 import os
+import re
 import sys
 
 import numpy as np
@@ -132,3 +133,11 @@ def quant_edge_rows():
     x = torch.from_numpy(rows).to(torch.bfloat16)
     assert torch.equal(x[0, :128].float(), torch.from_numpy(block.astype(np.float32)))
     return x
+
+
+def source_constant(file, name):
+    """An integer constant of the kernels' sources, so that a test of a rule follows it."""
+    with open(os.path.join(ROOT, "flashinfer_mlsys_amd", "csrc", file)) as f:
+        found = re.findall(rf"constexpr int {name} = (\d+);", f.read())
+    assert len(found) == 1, f"{name} in {file}"
+    return int(found[0])

@@ -6,7 +6,6 @@ Everything goes through libmoe_mi355x.so's C ABI via flashinfer_mlsys_amd.
 """
 import ctypes
 import os
-import re
 
 import numpy as np
 import pytest
@@ -16,7 +15,8 @@ import flashinfer_mlsys_amd as fm
 from flashinfer_mlsys_amd import workloads as wl
 from oracle import cpu_ref, np_ref
 
-from conftest import ATOL, RTOL, assert_close_bf16, bf16_bits_to_f32, golden_lists, load_golden, quant_edge_rows
+from conftest import ATOL, RTOL, assert_close_bf16, bf16_bits_to_f32, golden_lists, load_golden, quant_edge_rows, \
+    source_constant
 
 pytestmark = pytest.mark.gpu
 
@@ -467,19 +467,10 @@ def test_gemm2_item_heights_match_oracle(weights, dev, counts):
     assert_close_bf16(out, ref, f"counts={counts}")
 
 
-def _source_constant(file, name):
-    """An integer constant of the kernels' sources, so that a test of a rule follows it."""
-    path = os.path.join(os.path.dirname(fm.__file__), "csrc", file)
-    with open(path) as f:
-        found = re.findall(rf"constexpr int {name} = (\d+);", f.read())
-    assert len(found) == 1, f"{name} in {file}"
-    return int(found[0])
-
-
 def _takes_wide_gemm2(counts):
     """The rule of g2_takes_wide (csrc/moe_gemm.hip) for a call that both GEMM2 kernels are given."""
     tiles = sum((c + 255) // 256 for c in counts)
-    return sum(counts) >= _source_constant("moe_gemm.hip", "G2_WIDE_ROWS") * tiles
+    return sum(counts) >= source_constant("moe_gemm.hip", "G2_WIDE_ROWS") * tiles
 
 
 @pytest.mark.parametrize("counts,wide", [([40] * 32, False), ([75] * 31 + [74], False), ([75] * 32, True),
@@ -491,7 +482,7 @@ def test_gemm2_kernel_follows_the_rows_per_expert(weights, dev, counts, wide):
     loader GEMM2, which every call below runs: tokens are independent, so its output is
     then bit for bit that of the same tokens in two smaller calls. With more rows per
     256-row tile the wide kernel takes it, whose sums round differently."""
-    offset, line = 160, _source_constant("moe_capi.hip", "kWideMinTokens")
+    offset, line = 160, source_constant("moe_capi.hip", "kWideMinTokens")
     n = sum(counts)
     lg, b = _routing_for_counts(counts, offset, 3535 + n) if n else (torch.empty((0, 256)), None)
     T = line + 5
@@ -525,7 +516,7 @@ def test_wide_gemm2_row_counts_and_scales_match_oracle(weights, dev, scales):
     offset = 32
     lg, b = _routing_for_counts(counts, offset, 4949)
     T = lg.shape[0]
-    assert T >= _source_constant("moe_capi.hip", "kWideMinTokens") and _takes_wide_gemm2(counts)
+    assert T >= source_constant("moe_capi.hip", "kWideMinTokens") and _takes_wide_gemm2(counts)
     _say(f"wide GEMM2 T={T} scales={scales}")
     hs, hss = wl.quantize_1x128(wl.hidden_bf16(T, 4950).to(torch.float32))
     cpu_w = list(weights[0])

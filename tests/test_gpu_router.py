@@ -10,7 +10,7 @@ import flashinfer_mlsys_amd as fm
 from flashinfer_mlsys_amd import workloads as wl
 from oracle import cpu_ref, np_ref
 
-from conftest import assert_close_bf16
+from conftest import assert_close_bf16, source_constant
 
 pytestmark = pytest.mark.gpu
 
@@ -66,11 +66,19 @@ def test_router_deterministic_and_in_place(dev, gate, T):
     assert b is out and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("T", [1, 5, 16, 17, 64, 100, 575, 576, 1024, 3000])
+def _fused(T, dev):
+    """The rule of launch_router_quantize (csrc/moe_router.hip): one kernel, or two in turn."""
+    cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    return (T < source_constant("moe_router.hip", "RT2_MIN_T") or (T + 31) // 32 * 4 <= cu
+            or T >= source_constant("moe_router.hip", "RQ_MIN_TILED_T"))
+
+
+@pytest.mark.parametrize("T", [1, 5, 16, 17, 64, 100, 575, 576, 1024, 2049, 2999, 3000])
 def test_fused_producer_equals_separate_kernels(dev, gate, T):
     """router_logits_and_quantize writes the same logits, e4m3 rows and scales, bit
     for bit, as router_logits and quantize_activations (both kernels' tilings, ragged
     tiles); the rows and scales also equal the CPU oracle's quantiser."""
+    assert _fused(T, dev) == (T not in (2049, 2999))  # the two counts at the ends of the other branch
     print(f"fused producer T={T}", flush=True)
     x = wl.hidden_bf16(T, 300 + T)
     xd = x.to(dev)
@@ -83,12 +91,13 @@ def test_fused_producer_equals_separate_kernels(dev, gate, T):
         assert torch.equal(q.cpu().view(torch.uint8), qr.view(torch.uint8)) and torch.equal(s.cpu(), sr)
 
 
-@pytest.mark.parametrize("T", [577, 2047, 2048, 2304, 2433, 8191, 17001])
+@pytest.mark.parametrize("T", [577, 2047, 2048, 3000, 3073, 8191, 17001])
 def test_quantiser_waves_equal_the_quantiser_kernel(dev, gate, T):
     """The quantiser waves of the two tiled router kernels (whole and ragged token
     tiles, one and several items per workgroup) against the router and quantiser kernels
     alone, bit for bit, on values that leave the quick path too: zeros of both signs,
     tiny blocks, infinities and NaNs."""
+    assert _fused(T, dev)
     x = wl.hidden_bf16(T, 77).to(dev)
     x[0, :128] = 0
     x[1, 128:256] *= 1e-20
@@ -102,7 +111,7 @@ def test_quantiser_waves_equal_the_quantiser_kernel(dev, gate, T):
     assert torch.equal(lg.view(torch.int32), fm.router_logits(x, gate[1]).view(torch.int32))
 
 
-@pytest.mark.parametrize("T", [577, 2305, 2433])
+@pytest.mark.parametrize("T", [577, 2305, 2433, 3001, 3073])
 def test_producer_writes_nothing_past_its_outputs(dev, gate, T):
     """Ragged last token tiles: the outputs are the front of larger buffers (the rows of a
     whole tile and more behind them), whose tails stay as they were. The hidden states are
@@ -123,10 +132,12 @@ def test_producer_writes_nothing_past_its_outputs(dev, gate, T):
     assert torch.equal(out[0], fm.router_logits(x[:T], gate[1]))
 
 
-@pytest.mark.parametrize("T", [37, 700])
-def test_producer_graph_replay(dev, gate, T):
-    """The producer step (fused below 576 tokens, two kernels from 576) captured in a
-    HIP graph: each replay, with eager work in between, reproduces the eager result."""
+@pytest.mark.parametrize("T,fused", [(37, True), (700, True), (2500, False), (3073, True)])
+def test_producer_graph_replay(dev, gate, T, fused):
+    """The producer step (the small kernel, either tiled kernel with quantiser waves, and
+    the router and quantiser kernels in turn) captured in a HIP graph: each replay, with
+    eager work in between, reproduces the eager result."""
+    assert _fused(T, dev) == fused
     x = wl.hidden_bf16(T, 41).to(dev)
     bufs = (torch.empty((T, 256), device=dev), torch.empty((T, 7168), dtype=torch.float8_e4m3fn, device=dev),
             torch.empty((56, T), device=dev))
