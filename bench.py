@@ -6,7 +6,8 @@ intermediate 2048, 256 global experts, local experts 0-31, top-8 of 4-of-8
 groups, routed_scaling_factor 2.5) with seeded synthetic inputs. One step is one
 operator call at each T of the sweep, with every input resident in HBM.
 
-Printed JSON line (rank 0, one line):
+Printed JSON line (rank 0, one line of a few KB; --report FILE writes the same figures with
+every trial, stage time, byte count and error):
   value         tokens/s over the sweep = steps * sum(T) / wall time of the timed steps
                 (the step timed as a HIP graph replay and as plain API calls; the faster)
   ms_per_step   wall time of one sweep
@@ -27,7 +28,7 @@ Printed JSON line (rank 0, one line):
                 19 official trace workloads (T, offset) in the notebook's order, one row each
                 (us/call, binding roofline, P, E_act, CPU-oracle time); every configuration's
                 error over its whole output against the oracle's output (max abs, max rel, worst
-                err / (atol + rtol |ref|)); the drop-in
+                err / (atol + rtol |ref|); the line has the last alone); the drop-in
                 Python entry point timed at T=1 (host cost included); and the producer-side
                 kernels (FP8 activation quantiser, router GEMM, both fused) at T = 64 and 8192
 """
@@ -327,6 +328,36 @@ def mfma_pass(dev, weights_gpu, reps):
     print(json.dumps({"mfma_pass": True, "cases": info}), flush=True)
 
 
+def brief(out):
+    """The printed line: a few KB, so that a reader that keeps only the end of the output has all of
+    it. The headline fields whole, one short row per configuration."""
+    def err(row):
+        return (row.get("error_vs_oracle_full_output") or {}).get("max_err_over_bar")
+
+    def config(row):
+        return {"T": row["T"], "us_per_call": row["us_per_call"], "bound": row["roofline"]["bound"],
+                "frac": row["roofline"]["frac"], "cpu_oracle_us": row.get("cpu_oracle_us_per_call"),
+                "err_over_bar": err(row)}
+
+    b = {k: v for k, v in out.items() if k not in ("per_T", "also")}
+    b["per_T"] = [{"T": r["T"], "us_per_call": r["us_per_call"], "tokens_per_s": r["tokens_per_s"],
+                   "hbm_frac": r["hbm_frac"], "cold_us_per_call": r["cold_us_per_call"],
+                   "stage_us": list(r["stage_us"].values()), "err_over_bar": err(r)} for r in out["per_T"]]
+    also = {}
+    for name, row in out["also"].items():
+        if name == "official":  # T, offset, us, share of the binding roof, error over the bar
+            also[name] = [[r["T"], r["local_expert_offset"], r["us_per_call"], r["roofline"]["frac"], err(r)]
+                          for r in row]
+        elif "roofline" in row:
+            also[name] = config(row)
+        elif name == "dropin_kernel_T1":
+            also[name] = row
+        else:
+            also[name] = {T: r["us_per_call"] for T, r in row.items()}
+    b["also"] = also
+    return b
+
+
 def main():
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("--gpus", type=int, default=1)
@@ -335,6 +366,8 @@ def main():
     ap.add_argument("--reps", type=int, default=30, help="event-timed calls per T for per-kernel figures")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-extra", action="store_true", help="skip the prefill/skew summary")
+    ap.add_argument("--report", metavar="FILE", help="also write every figure (trials, stage times, byte counts, "
+                                                     "errors) as JSON to FILE")
     ap.add_argument("--traffic-pass", action="store_true",
                     help="only run the launches a rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE pass reads: a copy "
                          "kernel of known size, then --reps operator calls at each T of the sweep")
@@ -641,7 +674,10 @@ def main():
         "per_T": per_T,
         "also": also,
     }
-    print(json.dumps(out), flush=True)
+    if args.report:
+        with open(args.report, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(brief(out), separators=(",", ":")), flush=True)
 
 
 if __name__ == "__main__":
