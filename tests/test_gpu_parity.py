@@ -505,14 +505,39 @@ def test_gemm2_kernel_follows_the_rows_per_expert(weights, dev, counts, wide):
     assert err <= ATOL + RTOL * parts.float().abs().max().item()
 
 
-# W2 block scales for the wide GEMM2 (from 3,500 tokens): as made; one K block's scales 0 and one negative;
-# scales that differ by 2^44 within a row (both outside what its rescaled accumulators take).
-@pytest.mark.parametrize("scales", ["usual", "zero-negative", "far-apart"])
+WIDE_COUNTS = EDGE_COUNTS + [511, 513, 3, 240, 512]  # every number of row fragments of the wide GEMM2's items
+# W2 block scales for the wide GEMM2, which keeps its accumulators in units of the K block's scale where the
+# scales of a row lie within a factor of 2^40 (ratio) and scales every product where they do not, or are 0:
+# as made; signs that change from K block to K block; powers of two up to 2^-12 and up to 2^-39 times the
+# others, with changing signs, in K blocks that differ from row to row, the first and the last among them;
+# one K block's scales 0, one negative; scales that differ by 2^44.
+WIDE_SCALES = {"usual": True, "signs": True, "2^-12": True, "2^-39": True, "zero-negative": False, "far-apart": False}
+
+
+def _wide_scales(s2, kind):
+    s2 = s2.clone()
+    nb, kb = torch.meshgrid(torch.arange(s2.shape[1]), torch.arange(s2.shape[2]), indexing="ij")
+    sign = torch.where((nb + kb) % 3 == 0, -1.0, 1.0)
+    if kind == "signs":
+        s2 *= sign
+    elif kind.startswith("2^-"):  # at least half of a row's scales stay as made
+        low = int(kind[3:])
+        small = torch.where((kb + nb) % 4 == 0, 2.0 ** -low, torch.where((kb + nb) % 8 == 3, 2.0 ** -(low // 2), 1.0))
+        s2 *= sign * small
+    elif kind == "zero-negative":
+        s2[:, :, 3] = 0.0
+        s2[:, 1::2, 7] *= -1.0
+    elif kind == "far-apart":
+        s2[:, ::2, 5] *= 2.0 ** -44
+    return s2
+
+
+@pytest.mark.parametrize("scales", list(WIDE_SCALES))
 def test_wide_gemm2_row_counts_and_scales_match_oracle(weights, dev, scales):
-    """At 3,500 tokens and more GEMM2 takes 256-row items: experts with row counts at
-    the edges of its fragments, steps and tiles, with usual block scales and with
-    scales that take its general path, against the oracle."""
-    counts = EDGE_COUNTS + [511, 513, 3, 240, 512]
+    """From 3,500 tokens and 75 rows per tile GEMM2 takes 256-row items: experts with
+    row counts at the edges of its fragments, steps and tiles, with scales on both of
+    its paths, against the oracle."""
+    counts = WIDE_COUNTS
     offset = 32
     lg, b = _routing_for_counts(counts, offset, 4949)
     T = lg.shape[0]
@@ -520,30 +545,74 @@ def test_wide_gemm2_row_counts_and_scales_match_oracle(weights, dev, scales):
     _say(f"wide GEMM2 T={T} scales={scales}")
     hs, hss = wl.quantize_1x128(wl.hidden_bf16(T, 4950).to(torch.float32))
     cpu_w = list(weights[0])
-    s2 = cpu_w[3].clone()
-    if scales == "zero-negative":
-        s2[:, :, 3] = 0.0
-        s2[:, 1::2, 7] *= -1.0
-    elif scales == "far-apart":
-        s2[:, ::2, 5] *= 2.0 ** -44
-    cpu_w[3] = s2
+    s2 = cpu_w[3] = _wide_scales(cpu_w[3], scales)
+    # the kernel's test of a row of scales: within 2^40 of each other, nonzero
+    mag = s2.abs()
+    within = (mag.amin(dim=2) > 0) & (mag.amax(dim=2) * 9.0e-13 < mag.amin(dim=2))
+    assert bool(within.all()) if WIDE_SCALES[scales] else not bool(within[:, ::2].any())
     gpu = [t.to(dev) for t in (lg, b, hs, hss)] + list(weights[1])[:3] + [s2.to(dev)]
     out = fm.run(*gpu, offset, 2.5).float().cpu().numpy()
     ref = cpu_ref.run(lg, b, hs, hss, *cpu_w, offset, 2.5).float().numpy()
     assert_close_bf16(out, ref, f"wide GEMM2 scales={scales}")
 
 
-THIN_COUNTS = {"one-round-split-expert": [65, 64, 40, 33, 32, 1, 0, 17], "two-rounds": [7] * 19,
-               "two-rounds-split-experts": [66, 127, 64] + [5, 0, 33] * 8 + [1] * 4, "just-tiled": [6] * 24}
+def test_wide_gemm2_nan_and_saturated_rows(weights, dev):
+    """Rows of NaN and rows whose C exceeds fp16's range (it saturates) through the wide
+    GEMM2: the same NaNs and, within the bar, the same values as the loader GEMM2 gives
+    for the same tokens in two smaller calls, and every other row within it too."""
+    offset = 32
+    lg, b = _routing_for_counts(WIDE_COUNTS, offset, 5151)
+    T = lg.shape[0]
+    line = source_constant("moe_capi.hip", "kWideMinTokens")
+    assert T >= line and _takes_wide_gemm2(WIDE_COUNTS) and (T + 1) // 2 < line
+    _say(f"wide GEMM2 NaN and saturated rows T={T}")
+    hs, hss = wl.quantize_1x128(wl.hidden_bf16(T, 5152).to(torch.float32))
+    hss[5, 7::97] = float("nan")
+    hss[:, 11::89] *= 1e7
+    g = [t.to(dev) for t in (lg, b, hs, hss)]
+    whole = fm.run(*g, *weights[1], offset, 2.5).float().cpu()
+    half = T // 2
+    parts = torch.cat([fm.run(g[0][a:z].contiguous(), g[1], g[2][a:z].contiguous(), g[3][:, a:z].contiguous(),
+                              *weights[1], offset, 2.5) for a, z in ((0, half), (half, T))]).float().cpu()
+    nan = parts.isnan()
+    assert bool(nan[7::97].all()) and not bool(nan.all(dim=1).sum() > len(range(7, T, 97)))
+    assert torch.equal(whole.isnan(), nan)
+    big = torch.zeros(T, dtype=torch.bool)
+    big[11::89] = True
+    ok = ~nan.any(dim=1)
+    assert parts[big & ok].abs().max() > 1e5  # (usual outputs stay below 1e3)
+    assert_close_bf16(whole[ok & ~big].numpy(), parts[ok & ~big].numpy(), "usual rows")
+    # saturated rows: sums of terms far larger than themselves, against the row's own size
+    err = (whole - parts)[big & ok].norm(dim=1) / parts[big & ok].norm(dim=1)
+    assert float(err.max()) <= RTOL
+
+
+# (counts, whether the kernel takes thin items)
+THIN_COUNTS = {"one-round-split-expert": ([65, 64, 40, 33, 32, 1, 0, 17], True), "two-rounds": ([7] * 19, True),
+               "two-rounds-split-experts": ([66, 127, 64] + [5, 0, 33] * 6 + [1] * 3, True),
+               "tiled-split-experts": ([66, 127, 64] + [5, 0, 33] * 8 + [1] * 4, False), "just-tiled": ([6] * 24, False)}
+
+
+def _takes_thin_gemm1(counts, dev):
+    """The rule of gemm1_prefill_kernel (csrc/moe_gemm.hip)."""
+    grid = (torch.cuda.get_device_properties(dev).multi_processor_count + 7) // 8 * 8
+    rows, tiles_n = source_constant("moe_gemm.hip", "TH_ROWS"), 16
+    active = sum(c > 0 for c in counts)
+    slices = sum((c + rows - 1) // rows for c in counts)
+    rounds = -(-sum((c + 255) // 256 for c in counts) * tiles_n // grid)
+    if slices == 0 or slices > active + active // 4:
+        return False
+    return 10 * tiles_n * slices < 9 * grid if rounds == 1 else 4 * tiles_n * slices < 3 * rounds * grid
 
 
 @pytest.mark.parametrize("name", list(THIN_COUNTS))
 def test_thin_gemm1_items_match_oracle(weights, dev, name):
     """The prefill GEMM1 streams the weights (thin items) when few experts are active
     and nearly all have at most 64 rows: experts of 1 to 64 rows and of 65 to 127 (two
-    slices), one and two rounds of the tiled items, and 24 experts, which it leaves to
+    slices, in one and in two rounds of the tiled items), and counts that it leaves to
     the tiled items, against the oracle."""
-    counts, offset = THIN_COUNTS[name], 96
+    (counts, thin), offset = THIN_COUNTS[name], 96
+    assert _takes_thin_gemm1(counts, dev) == thin
     lg, b = _routing_for_counts(counts, offset, 7171 + sum(counts))
     T = lg.shape[0]
     assert T > 96
@@ -553,6 +622,29 @@ def test_thin_gemm1_items_match_oracle(weights, dev, name):
     out = fm.run(*gpu, offset, 2.5).float().cpu().numpy()
     ref = cpu_ref.run(lg, b, hs, hss, *weights[0], offset, 2.5).float().numpy()
     assert_close_bf16(out, ref, f"thin GEMM1 {name}")
+
+
+def test_thin_gemm1_items_in_a_short_last_chunk(weights, dev):
+    """A chunked call whose last chunk takes thin items: its activation scales lie in
+    rows of the whole call's length. Bit for bit the separate call on those tokens."""
+    from flashinfer_mlsys_amd import _lib
+    C, offset = _lib.MOE_FP8_CHUNK_TOKENS, 96
+    counts = THIN_COUNTS["two-rounds-split-experts"][0]
+    assert _takes_thin_gemm1(counts, dev)
+    tail, b = _routing_for_counts(counts, offset, 8181)
+    n = tail.shape[0]
+    lg = torch.full((C + n, 256), -8.0)
+    lg[:C, 128:136] = 6.0 + 0.1 * torch.arange(8)  # experts of another rank
+    lg[C:] = tail
+    _say(f"thin GEMM1 in a last chunk of {n} tokens")
+    hs, hss = wl.quantize_1x128(wl.hidden_bf16(C + n, 8282).to(torch.float32))
+    g = [t.to(dev) for t in (lg, b, hs, hss)]
+    out = fm.run(*g, *weights[1], offset, 2.5)
+    alone = fm.run(g[0][C:].contiguous(), g[1], g[2][C:].contiguous(), g[3][:, C:].contiguous(), *weights[1], offset, 2.5)
+    assert bool((out[:C] == 0).all())
+    assert torch.equal(out[C:].view(torch.int16), alone.view(torch.int16))
+    ref = cpu_ref.run(lg[C:], b, hs[C:], hss[:, C:].contiguous(), *weights[0], offset, 2.5).float().numpy()
+    assert_close_bf16(alone.float().cpu().numpy(), ref, "last chunk")
 
 
 DECODE_EDGE_COUNTS = [[64], [33, 31], [17, 16, 15, 1, 0, 15], [1] * 32, [0] * 31 + [48], [2, 3, 4, 5, 6, 7, 8, 9],
@@ -617,10 +709,12 @@ def test_dps_writes_into_output(case):
     assert_close_bf16(out.float().cpu().numpy()[case.g["out_rows"]], ref, "dps")
 
 
-@pytest.mark.parametrize("case", ["decode_t1", "decode_t8", "t16", "decode_t32", "prefill_t1024"], indirect=True)
+@pytest.mark.parametrize("case", ["decode_t1", "decode_t8", "t16", "decode_t32", "prefill_t1024", "skew_t4096"],
+                         indirect=True)
 def test_graph_replay_matches_eager(case):
-    """The forward captured in a HIP graph: every replay, with eager work and
-    synchronisations between replays, gives the eager output bit for bit."""
+    """The forward captured in a HIP graph (skew_t4096: with the wide GEMM2): every
+    replay, with eager work and synchronisations between replays, gives the eager
+    output bit for bit."""
     out = torch.empty((case.w.T, 7168), dtype=torch.bfloat16, device=case.gpu[0].device)
     ws = torch.empty(fm.workspace_size(case.w.T), dtype=torch.uint8, device=out.device)
     fm.kernel(*case.gpu, case.offset, case.rsf, out, workspace=ws)

@@ -22,7 +22,7 @@ from flashinfer_mlsys_amd import _lib
 BUNDLE_MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 EXPECTED = ("route_kernel", "route_count_kernel", "dispatch_count_kernel", "dispatch_scatter_kernel",
             "dispatch_small_kernel", "gemm1_decode_kernel", "gemm2_decode_kernel", "gemm1_prefill_kernel",
-            "gemm2_loader_kernel", "combine_kernel", "quantize_1x128_kernel", "router_small_kernel",
+            "gemm2_loader_kernel", "gemm2_wide_kernel", "combine_kernel", "quantize_1x128_kernel", "router_small_kernel",
             "router_tiled_kernel", "router_ksplit_kernel")
 SCRATCH_ALLOWED = {"gemm2_loader_kernel": 64}
 
