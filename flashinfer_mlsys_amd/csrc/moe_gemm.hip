@@ -691,8 +691,8 @@ __global__ __launch_bounds__(64 * D2_WAVES, 2) void gemm2_decode_kernel(
 // ---------------------------------------------------------------------------
 // Items of the tiled (prefill) kernels: (row tile, column tile) pairs.
 //
-// Row tiles are BM rows of one expert's segment (GEMM1: 256, GEMM2: 128),
-// numbered expert by expert in descending order of the experts' row counts
+// Row tiles are BM rows of one expert's segment (GEMM1 and the wide GEMM2: 256,
+// the loader GEMM2: 128 or 64), numbered expert by expert in descending order of the experts' row counts
 // (ties: lower id first), each expert's tiles in row order. All tiles of an
 // expert share its weight tiles, which stay in the caches while they run; the
 // largest experts (whose tiles are full and cost the most: the waves skip row
@@ -831,8 +831,8 @@ constexpr int FRAG_BYTES = 2048;
 //
 // Measured (GEMM1 alone, us, against the version that loaded a whole block between
 // two barriers and read each block's fragments after its barrier): skewed T=4096
-// (24.7k pairs, 227 rows a tile) 807 -> 660, T=14,107 571 -> 498, T=8192 393 -> 331,
-// T=3001 218 -> 191, T=901 165 -> 165 (5.7 TB/s of weights). On full tiles a block
+// (24.7k pairs, 227 rows a tile) 808 -> 715, T=14,107 573 -> 526, T=8192 375 -> 336,
+// T=3001 205 -> 189, T=901 165 -> 164 (5.7 TB/s of weights). On full tiles a block
 // takes 3,000 clk (2,176 of MFMAs; 2,950 with every MFMA taken out, the load path's
 // ~22 B/clk per CU), and the clock falls to 1.9-2.0 GHz: MFMAs alone on such data
 // run at 3.7 PFLOP/s, the card's power limit.
@@ -1612,15 +1612,15 @@ constexpr int Q2_A_BYTES = Q2_BM * BLK * 2;  // 32 KB: 4 row blocks x 2 lines
 constexpr int Q2_B_BYTES = Q2_BN * BLK;      // 32 KB: 8 row blocks
 constexpr int Q2_STAGE = Q2_A_BYTES + Q2_B_BYTES;
 
-
-
 // ---------------------------------------------------------------------------
 // GEMM2 kernel: the item, stage layout and K order above, with the global ->
 // LDS traffic (64 load instructions per K block, 16 per loader wave: waves 0-1
 // the activation rows, 2-3 the W2 rows) issued by 4 loader waves while the 8
-// compute waves read LDS, widen W2 and run MFMAs (as in GEMM1, a wave that
-// issues loads would hold back its MFMAs while the memory pipeline is busy). The two 64 KB slots run on across items: after K block kb's barrier
-// the loaders fill the other slot with block kb + 1 (of this item or the next).
+// compute waves read LDS, widen W2 and run MFMAs (a wave that issues loads holds
+// back its MFMAs while the CU's load path is busy; GEMM1 and the wide GEMM2 spread
+// theirs over the MFMAs instead). The two 64 KB slots run on across items: after
+// K block kb's barrier the loaders fill the other slot with block kb + 1 (of this
+// item or the next).
 // The last loader wave also carries the block's two W2 block scales (output
 // column blocks 2 nt and 2 nt + 1) into the stage.
 // ---------------------------------------------------------------------------
@@ -1971,10 +1971,10 @@ __global__ __launch_bounds__(W2_THREADS, 1) void gemm2_loader_kernel(
 // an activation row's half. W2's chunks are placed at position 2 g + h so that both kinds
 // of fragment read are free of bank conflicts.
 //
-// Measured against the loader kernel (whole calls, us): skewed T=4096 1,500 -> 1,400,
-// T=14,107 1,086 -> 1,005, T=4096 451 -> 430; GEMM2 alone at T=2500 151 -> 162, T=2000
-// 129 -> 137, T=901 101 -> 126: most experts there have fewer than 80 rows, whose
-// half-empty items cost more than the loader kernel's 64- and 128-row ones.
+// Measured against the loader kernel (GEMM2 alone, us): skewed T=4096 772 -> 665, T=14,107
+// 450 -> 407, T=8192 327 -> 292, T=4096 182 -> 167; but T=2500 151 -> 162, T=2000 129 -> 137,
+// T=901 101 -> 126: most experts there have fewer than 80 rows, whose half-empty items
+// cost more than the loader kernel's 64- and 128-row ones.
 // A block takes 5,650 clk on full items (4,608 of MFMAs).
 // ---------------------------------------------------------------------------
 constexpr int W_BM = 256, W_BN = 256;

@@ -15,7 +15,8 @@ namespace moe {
 __device__ __forceinline__ float qblock_scale(float amax) { return fmaxf(amax, 1e-12f) / 448.0f; }
 
 // x / s, correctly rounded, for a bf16 value x and its block's scale s: q = x y with y
-// within 3 ulps of 1 / s, then one residual step, q + y (x - s q) in fused operations.
+// within 3 ulps of 1 / s, then one residual step, q + y (x - s q) in fused operations (the
+// correction step of Markstein's division for machines with a fused multiply-add, 1990).
 // That is the correctly rounded quotient for every pair of a bf16 maximum and a bf16
 // value (their 128 x 128 significands, checked one by one: the steps scale exactly with
 // the exponents, and a quotient that does not round to the code 0 has |q| >= 2^-10 and

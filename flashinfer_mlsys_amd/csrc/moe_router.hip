@@ -21,7 +21,7 @@
 // Larger T: LDS-staged tiles of 128 tokens x 64 experts, 8 compute waves of
 // 32 x 32 (v_mfma_f32_32x32x16_bf16) and 4 loader waves that stream each 128-wide
 // K block (hidden rows and gate rows, whole 128 B lines, 32-row swizzle) into a
-// 3-slot LDS ring two blocks ahead, as the prefill GEMM1 does. Between 576 tokens
+// 3-slot LDS ring two blocks ahead. Between 576 tokens
 // and the token count whose 32-token items fill the CUs once (2,048 on 256 CUs),
 // router_ksplit_kernel: 32 x 64 tiles, a 5-slot ring, each K block's MFMA steps
 // split over the 8 compute waves and the four K quarters added in LDS in a
