@@ -2035,6 +2035,9 @@ __device__ __forceinline__ WSrc w_src(const WCtx& x, const WItem& it, bool have)
 }
 
 // This wave's loads of activation unit (kb, q): rows 128 (q % 2) + 16 w .., K half q / 2.
+// (Rows past the item's valid ones: their sums are dropped, and whether or not the range check
+// covers the scalar offset, which holds the 16-row step, they lie in the workspace: at most 255
+// rows of 4 KB past the pair rows' C, where the partial rows follow.)
 __device__ __forceinline__ void w_load_a(const WCtx& x, v4i rs, int kb, int q, int slot) {
   const uint32_t so = (uint32_t)((q & 1) * 128 + 16 * x.w) * (I * 2) + kb * 256 + (q >> 1) * 128;
   const uint32_t d = x.l0 + slot * W_AREG + x.w * 2048;
